@@ -25,16 +25,22 @@
 //
 // Cache layout: k_cache, v_cache (batch, n_kv, cap, 128) fp16, the
 // reference's (B, n_kv, S, D) tensors with room for cap positions.
+#include "attn_kernels.h"
 #include "capi_util.h"
 #include "decode_util.h"
+#include "ffn_kernels.h"
 
 namespace oi2 {
 namespace {
 
-constexpr int kHd = 128;                 // head_dim (engine.py:72: hidden / n_q)
+constexpr int kHd = kHeadDim;
 constexpr int kHalf = kHd / 2;
-constexpr int kThreads = 256;
 constexpr int kMaxRows = 8;              // token rows per GEMV launch
+// From these rows on the projections run on the matrix cores (attn_prompt.hip):
+// the GEMV takes 17.2 + 8.2 us per 8 rows (q / k / v and o_proj), k_rmsnorm and
+// k_proj 3 + 18 + 16 us from 9 rows to 64.
+constexpr int kPromptRows = 9;
+constexpr int kPromptMaxRows = 0x7FFFFFFF / (kH * 2);   // 32-bit byte offsets into the rows
 constexpr int kMinPosPerWg = 32;         // 4 waves x 2 steps of 4 positions
 constexpr int kMaxTabBytes = 64 << 10;   // the merge's m / l table in LDS
 
@@ -812,7 +818,38 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
   g.cos = cos;
   g.sin = sin;
   g.n_counters = rows * n_kv;
-  for (int r0 = 0; r0 < rows; r0 += kMaxRows) {
+  const bool prompt = rows >= kPromptRows && rows <= kPromptMaxRows;
+  if (prompt) {
+    // x_n into the attention output's buffer, free until the attention runs
+    hipLaunchKernelGGL(k_rmsnorm, dim3(rows), dim3(kThreads), 0, st, x, w->norm_w, eps, attn);
+    OI2_CHECK_LAUNCH();
+    ProjArgs p{};
+    p.x = attn;
+    p.rows = rows;
+    p.w0 = w->wq;
+    p.w1 = w->wk;
+    p.w2 = w->wv;
+    p.blocks0 = n_q;
+    p.blocks1 = n_kv;
+    p.mode = 0;
+    p.q = qb;
+    p.q_width = n_q * kHd;
+    p.k_cache = k_cache;
+    p.v_cache = v_cache;
+    p.n_kv = n_kv;
+    p.cap = cache_cap;
+    p.past = past;
+    p.seq = seq;
+    p.cos = cos;
+    p.sin = sin;
+    launch_proj(p, n_q + 2 * n_kv, st);
+    OI2_CHECK_LAUNCH();
+    if (past + seq > kOneWgMax) {
+      hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(kThreads), 0, st, counters, rows * n_kv, 0u);
+      OI2_CHECK_LAUNCH();
+    }
+  }
+  for (int r0 = 0; !prompt && r0 < rows; r0 += kMaxRows) {
     const int rc = rows - r0 < kMaxRows ? rows - r0 : kMaxRows;
     g.x = x + (size_t)r0 * kH;
     g.row0 = r0;
@@ -853,6 +890,21 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
     OI2_CHECK_LAUNCH();
   }
 
+  if (prompt) {
+    ProjArgs p{};
+    p.x = attn;
+    p.rows = rows;
+    p.w0 = w->wo;
+    p.blocks0 = kH / kHd;
+    p.mode = 1;
+    p.seq = seq;
+    p.out = out;
+    p.residual = x_out ? x : nullptr;
+    p.x_out = x_out;
+    launch_proj(p, kH / kHd, st);
+    OI2_CHECK_LAUNCH();
+    return OI2_OK;
+  }
   GemvArgs o{};
   o.norm_w = nullptr;
   o.w0 = w->wo;

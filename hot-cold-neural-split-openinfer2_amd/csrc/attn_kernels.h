@@ -1,0 +1,37 @@
+// Argument blocks shared by the attention sources: the single-token kernels
+// (attention.hip) and the prompt kernels (attn_prompt.hip).
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace oi2 {
+
+constexpr int kHeadDim = 128;                 // head_dim (engine.py:72: hidden / n_q)
+
+// Rows of x times weight blocks of 128 rows (one head each): q / k / v with
+// RoPE, q to a buffer and k, v into the cache (mode 0), or o_proj (mode 1).
+struct ProjArgs {
+  const uint16_t* x;          // input rows (rows, H) fp16
+  int rows;
+  const uint8_t* w0;          // weight blocks of 128 rows (.., H), fp8 e4m3fn
+  const uint8_t* w1;
+  const uint8_t* w2;
+  int blocks0, blocks1;       // 128-row blocks in w0 and w1; the rest are w2's
+  int mode;
+  // mode 0
+  uint16_t* q;                // (rows, n_q * 128)
+  int q_width;                // n_q * 128
+  uint16_t* k_cache;
+  uint16_t* v_cache;
+  int n_kv, cap, past, seq;
+  const float* cos;           // (seq, 64)
+  const float* sin;
+  // mode 1
+  uint16_t* out;              // (rows, H)
+  const uint16_t* residual;   // (rows, H) or null
+  uint16_t* x_out;
+};
+
+void launch_proj(const ProjArgs& a, int n_heads, hipStream_t st);
+
+}  // namespace oi2

@@ -1963,7 +1963,7 @@ static BatchPlan batch_plan(int M, int n_hot, int cap) {
 }
 
 // The current device's CU count (cached per device).
-static int device_cus() {
+int device_cus() {
   static int cache[64] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;

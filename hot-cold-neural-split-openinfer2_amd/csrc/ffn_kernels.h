@@ -222,6 +222,7 @@ __global__ void k_bup(BUpArgs a);
 __global__ void k_rmsnorm(const uint16_t* x, const uint16_t* w, float eps, uint16_t* out);
 
 size_t batch_ws_bytes(int M, int n_hot, int cap);
+int device_cus();   // the current device's CU count
 // Scratch carve-up of the single-token decode FFN (k_prep / k_ffn_up /
 // k_ffn_down): h_hot, cold partial rows (one per cold workgroup), the cold
 // item total, x * w and the norm's sum-of-squares partials.

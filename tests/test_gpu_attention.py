@@ -220,3 +220,19 @@ def test_rewind_decodes_a_position_again_in_place(dev):
         assert torch.equal(t, s)
     with pytest.raises(ValueError):
         attn.rewind(12)
+
+
+@pytest.mark.parametrize("B,T,n_kv", [(1, 9, 8), (1, 63, 32), (1, 64, 8), (2, 65, 4), (1, 129, 8), (3, 43, 16),
+                                      (1, 400, 8), (1, 700, 32), (11, 1, 8)])
+def test_prompt_rows_on_the_matrix_cores(dev, B, T, n_kv):
+    """Rows at the edges of the prompt projections' 64- and 128-row tiles and
+    of their choice of tile (400 rows with 48 heads and 700 rows with 96 fill
+    more than one tile per CU), several sequences with rows of each in one
+    tile, a batch of single rows over a cache."""
+    w = _weights(dev, n_kv, seed=51 + T)
+    attn = oi2.GroupedQueryAttention(0, w, _cfg(n_kv))
+    past = 33 if T == 1 else 0
+    cos, sin = oi2.rope_tables(past + T, D, 1e6, device=dev)
+    x = torch.randn((B, T, H), generator=torch.Generator(device=dev).manual_seed(52), device=dev).half()
+    cache = _rand_cache(dev, B, n_kv, past, seed=53) if past else None
+    _check_step(attn, w, n_kv, x, cos[past:], sin[past:], cache, f"prompt B={B} T={T} n_kv={n_kv}")
