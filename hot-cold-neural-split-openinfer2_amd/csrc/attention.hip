@@ -1,7 +1,8 @@
 // Grouped-query attention for decode on gfx950: GroupedQueryAttention.forward
 // (engine.py:90-125) with the KV cache kept in place.
 //
-// One call runs three kernels on its stream:
+// One call runs three kernels on its stream (with 9 and more token rows k_proj
+// and, for rows enough, k_flash of attn_prompt.hip, k_rmsnorm ahead of them):
 //   k_attn_gemv (qkv)  RMSNorm of the token rows (input_layernorm,
 //                      engine.py:93), then q, k, v = fp16(x_n W^T) from the
 //                      fp8 e4m3fn weights (the reference keeps them fp8 at
@@ -40,6 +41,8 @@ constexpr int kMaxRows = 8;              // token rows per GEMV launch
 // the GEMV takes 17.2 + 8.2 us per 8 rows (q / k / v and o_proj), k_rmsnorm and
 // k_proj 3 + 18 + 16 us from 9 rows to 64.
 constexpr int kPromptRows = 9;
+constexpr int kFlashSeq = 9;             // rows of a sequence from which attention runs on the matrix cores
+constexpr int kFlashMaxSpan = 1 << 23;   // 32-bit byte offsets into one head's cache
 constexpr int kPromptMaxRows = 0x7FFFFFFF / (kH * 2);   // 32-bit byte offsets into the rows
 constexpr int kMinPosPerWg = 32;         // 4 waves x 2 steps of 4 positions
 constexpr int kMaxTabBytes = 64 << 10;   // the merge's m / l table in LDS
@@ -819,6 +822,13 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
   g.sin = sin;
   g.n_counters = rows * n_kv;
   const bool prompt = rows >= kPromptRows && rows <= kPromptMaxRows;
+  // The prompt attention walks the span in one workgroup per 64 rows and head.
+  // A handful of rows over a long span has too few of those, and the split
+  // kernel is faster (whole layer, n_kv 8: 9 rows over 1000 positions 49 us
+  // against 52, over 4000 73 against 90; 16 rows over 4000 102 against 91,
+  // 64 rows 382 against 94; n_kv 32: 9 rows over 4000 149 against 91).
+  const bool flash = prompt && seq >= kFlashSeq && past + seq <= kFlashMaxSpan &&
+                     (rows >= 16 || rows * n_kv >= 256 || past + seq <= 512);
   if (prompt) {
     // x_n into the attention output's buffer, free until the attention runs
     hipLaunchKernelGGL(k_rmsnorm, dim3(rows), dim3(kThreads), 0, st, x, w->norm_w, eps, attn);
@@ -844,7 +854,7 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
     p.sin = sin;
     launch_proj(p, n_q + 2 * n_kv, st);
     OI2_CHECK_LAUNCH();
-    if (past + seq > kOneWgMax) {
+    if (past + seq > kOneWgMax && !flash) {
       hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(kThreads), 0, st, counters, rows * n_kv, 0u);
       OI2_CHECK_LAUNCH();
     }
@@ -869,7 +879,22 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
   s.causal = causal ? 1 : 0;
   s.scale = 1.0f / sqrtf((float)kHd);
   s.out = attn;
-  if (past + seq <= kOneWgMax) {
+  if (flash) {
+    FlashArgs f{};
+    f.q = qb;
+    f.k_cache = k_cache;
+    f.v_cache = v_cache;
+    f.n_kv = n_kv;
+    f.cap = cache_cap;
+    f.past = past;
+    f.seq = seq;
+    f.batch = batch;
+    f.causal = causal ? 1 : 0;
+    f.scale = s.scale;
+    f.out = attn;
+    launch_flash(f, st);
+    OI2_CHECK_LAUNCH();
+  } else if (past + seq <= kOneWgMax) {
     // short spans: the whole span in one workgroup per (row, query head)
     s.n_split = 1;
     launch_sdpa1(s, G, rows, st);

@@ -34,4 +34,16 @@ struct ProjArgs {
 
 void launch_proj(const ProjArgs& a, int n_heads, hipStream_t st);
 
+// Attention of (batch, seq) query rows over cache positions [0, past + seq).
+struct FlashArgs {
+  const uint16_t* q;          // (batch * seq, H)
+  const uint16_t* k_cache;    // (batch, n_kv, cap, 128)
+  const uint16_t* v_cache;
+  int n_kv, cap, past, seq, batch, causal;
+  float scale;
+  uint16_t* out;              // (batch * seq, H)
+};
+
+void launch_flash(const FlashArgs& a, hipStream_t st);
+
 }  // namespace oi2

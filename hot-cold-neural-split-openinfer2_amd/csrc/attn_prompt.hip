@@ -5,6 +5,8 @@
 //   k_proj       C = X W^T, fp16 rows times fp8 e4m3fn weights (widened
 //                exactly to fp16), fp32 sums; epilogue q / k / v (RoPE, q to a
 //                buffer, k and v into the cache) or o_proj (out and x + out)
+//   k_flash      attention of 64 query rows of a head per workgroup over the
+//                cache positions they see
 //
 // Rounded to fp16: x_n, q, k, v before and after RoPE, the attention output
 // and out; everything between them is fp32.
@@ -309,6 +311,297 @@ __global__ __launch_bounds__(256, KB == 64 ? 2 : 1) void k_proj(ProjArgs a, int 
   }
 }
 
+// ── attention ────────────────────────────────────────────────────────────────
+//
+// Workgroup: 64 query rows of one head over the positions they see, 32 NK a
+// tile, 2 NK waves.  Wave (qs, kv) = (w & 1, w >> 1) takes query rows 32 qs ..
+// and the kv-th 32 positions of every tile with its own running max, sum and
+// output (flash-style); the NK position parts meet in LDS at the end.
+//
+// The scores are taken transposed, S^T = K Q^T (32x32x16 MFMAs), so that a
+// lane holds 16 scores of ONE query (column l % 32): max, sum and rescaling
+// are per lane, one exchange with lane l ^ 32 for the max.  Element j of lane
+// half h is position 8 (j / 4) + 4 h + j % 4; out^T += V^T P^T takes the
+// probabilities as they lie, K step s the elements 8 s .. 8 s + 7, with the
+// positions of V^T stored in that order.
+//
+// Probabilities stay 32-bit: p 2^10 = hi + lo in two fp16 parts (hi truncated,
+// lo the rest, at least 21 bits; the 2^10 keeps lo of small p out of the
+// subnormals and cancels in the division by the sum), two MFMAs per fragment.
+//
+// What bounds it: the chain of one tile (scores, max, probabilities, output:
+// 24 MFMAs and ~200 vector instructions a wave) and, causal, the longest row
+// tile's chain of tiles.  512 rows 17 us (one workgroup per query row and
+// head, the single-token kernel: 134), 1300 rows 38 us (split kernel: 1078).
+// Reading a tile's eight K fragments ahead of its MFMAs changed nothing.
+//
+// K goes to LDS by DMA; V through registers, 4 positions x 8 dims a thread,
+// transposed to rows of one dim.  Both two buffers, one barrier per tile.
+constexpr int kFQ = 64;                        // query rows per workgroup
+constexpr float kLog2e = 1.44269504088896341f;
+
+// Byte offset of 16-byte chunk c (8 positions) of V^T's row d.  The transposed
+// stores (rows 8 apart) and the fragment reads (16 consecutive rows) both
+// spread over all banks.
+template <int NK>
+__device__ __forceinline__ int vt_off(int d, int c) {
+  if (NK == 4) return d * 256 + 16 * (c ^ (((d >> 3) ^ d) & 15));
+  return (d ^ ((d >> 3) & 1)) * 128 + 16 * (c ^ (((d >> 4) ^ (d >> 1)) & 7));
+}
+
+__device__ __forceinline__ bool f16_nonfinite(uint32_t h) { return (h & 0x7C00u) == 0x7C00u; }
+
+template <int NK>
+__global__ __launch_bounds__(128 * NK, 4 / NK) void k_flash(FlashArgs a, int n_qt) {
+  constexpr int kFP = 32 * NK;                 // positions per tile
+  constexpr int kW = 2 * NK;                   // waves
+  __shared__ __align__(1024) uint8_t sK0[kFP * 256], sK1[kFP * 256];
+  __shared__ __align__(1024) uint8_t sV0[kHeadDim * kFP * 2], sV1[kHeadDim * kFP * 2];
+  __shared__ float s_m[kW][32], s_l[kW][32];
+  __shared__ uint32_t s_bad[2][NK];            // per buffer: positions of the tile with a non-finite v
+  const int b = blockIdx.x;
+  // the four heads of blocks 8 apart share an XCD: with up to 8 kv heads they
+  // are of one kv head, whose K and V its L2 then holds
+  const int hq = (b & 7) * (kH / kHeadDim / 8) + ((b >> 3) & 3), rest = b >> 5;
+  const int bt = rest / n_qt, q0 = (n_qt - 1 - rest % n_qt) * kFQ;   // the longest rows first
+  const int g = hq / (kH / kHeadDim / a.n_kv);
+  const int t = threadIdx.x, l = lane_id(), r = l & 31, h = l >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6), qs = w & 1, kv = w >> 1;
+  const int n_pos = a.past + a.seq;
+  const int n_see = a.causal ? min(a.past + q0 + kFQ, n_pos) : n_pos;   // positions this workgroup reads
+  const int n_kt = (n_see + kFP - 1) / kFP;
+
+  const size_t head = ((size_t)bt * a.n_kv + g) * a.cap * kHeadDim;
+  const rsrc_t rk = rsrc(a.k_cache + head, (uint32_t)n_pos * 256);
+  const rsrc_t rv = rsrc(a.v_cache + head, (uint32_t)n_pos * 256);
+  // K DMA i: rows 4 (w + kW i) + l / 16, chunk l % 16
+  uint32_t koff[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 4 * (w + kW * i) + (l >> 4);
+    koff[i] = (uint32_t)row * 256 + 16 * swz<16>(row, l & 15);
+  }
+  // V: positions 4 (t / 16) .. + 3, dims 8 (t % 16) .. + 7
+  const int pg = t >> 4, dc = t & 15;
+  const uint32_t voff = (uint32_t)(4 * pg) * 256 + 16 * dc;
+  const int og = (pg >> 2) * 4 + (pg & 1) * 2 + ((pg >> 1) & 1);   // its 4-position group in V^T's order
+  u32x4 vr[4];
+  auto load_k = [&](int kt, uint8_t* sK) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dma16(rk, sK + 1024 * (w + kW * i), koff[i] + (uint32_t)kt * (kFP * 256), 0);
+  };
+  auto load_v = [&](int kt) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) vr[i] = bld16(rv, voff + (uint32_t)kt * (kFP * 256) + 256 * i);
+  };
+  // whether some row of the workgroup must not see some position of tile kt
+  auto masked = [&](int kt) { return a.causal && (kt + 1) * kFP > a.past + q0 + 1; };
+  auto store_v = [&](int kt, int buf, uint8_t* sV) {
+    if (masked(kt)) {
+      // a masked position's probability is 0, and 0 times a non-finite v would
+      // spoil rows that do not see it: such v go in as 0 here, and their
+      // positions are noted and added one by one to the rows that see them
+      uint32_t bad = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const uint32_t x = vr[i][d];
+          const uint32_t lo = f16_nonfinite(x) ? 0xFFFFu : 0u, hi = f16_nonfinite(x >> 16) ? 0xFFFF0000u : 0u;
+          vr[i][d] = x & ~(lo | hi);
+          if (lo | hi) bad |= 1u << i;
+        }
+      if (bad) atomicOr(&s_bad[buf][pg >> 3], bad << (4 * (pg & 7)));
+    }
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const uint32_t x0 = vr[0][d], x1 = vr[1][d], x2 = vr[2][d], x3 = vr[3][d];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const uint32_t sel = k ? 0x07060302u : 0x05040100u;
+        const int row = 8 * dc + 2 * d + k;
+        *reinterpret_cast<u32x2v*>(sV + vt_off<NK>(row, og >> 1) + 8 * (og & 1)) =
+            u32x2v{__builtin_amdgcn_perm(x1, x0, sel), __builtin_amdgcn_perm(x3, x2, sel)};
+      }
+    }
+  };
+
+  // this lane's query row, all 128 dims: B operand, K step st dims 16 st + 8 h
+  const int tq = q0 + 32 * qs + r;                        // row within the sequence
+  const int tc = tq < a.seq ? tq : a.seq - 1;             // rows past it repeat the last one, not stored
+  const uint16_t* pq = a.q + ((size_t)bt * a.seq + tc) * kH + hq * kHeadDim + 8 * h;
+  h8 qf[8];
+#pragma unroll
+  for (int st = 0; st < 8; ++st) qf[st] = *reinterpret_cast<const h8*>(pq + 16 * st);
+  const int lim = a.causal ? a.past + tc + 1 : n_pos;     // positions this row sees
+  const float sc2 = a.scale * kLog2e;
+  const float ninf = -__builtin_inff();
+
+  f32x16 o[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) o[d] = f32x16{};
+  float m = ninf, lsum = 0.0f;                            // of this lane's positions; m of both halves
+
+  if (t < 2 * NK) s_bad[t / NK][t % NK] = 0;
+  load_k(0, sK0);
+  load_v(0);
+  __syncthreads();                                        // s_bad is cleared
+  store_v(0, 0, sV0);
+
+  auto tile = [&](int kt, int buf, const uint8_t* cK, const uint8_t* cV, uint8_t* nK, uint8_t* nV) {
+    // K's DMAs (the only loads in flight) and V's stores of this tile are done
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const bool more = kt + 1 < n_kt;
+    if (more) {
+      load_k(kt + 1, nK);
+      load_v(kt + 1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int p0 = kt * kFP + 32 * kv;                    // this wave's first position
+    const bool live = p0 < n_see;
+    if (live) {
+      f32x16 s = {}, s1 = {};                             // two chains: an MFMA's result takes a while
+#pragma unroll
+      for (int st = 0; st < 8; ++st) {
+        const int row = 32 * kv + r;
+        const h8 kf = *reinterpret_cast<const h8*>(cK + row * 256 + 16 * swz<16>(row, 2 * st + h));
+        if (st & 1) s1 = mfma32(kf, qf[st], s1);
+        else s = mfma32(kf, qf[st], s);
+      }
+      s += s1;
+      if (masked(kt) || p0 + 32 > n_pos) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const int p = p0 + 8 * (j >> 2) + 4 * h + (j & 3);
+          s[j] = p < lim ? s[j] : ninf;
+        }
+      }
+      float cm = s[0];
+#pragma unroll
+      for (int j = 1; j < 16; ++j) cm = fmaxf(cm, s[j]);
+      cm = fmaxf(cm, __shfl_xor(cm, 32)) * sc2;
+      // The sums are taken against m, which follows the row's max only once
+      // that is 2^5 above it (p 2^10 stays within fp16's range): most tiles
+      // then skip the 65 products of the rescaling.
+      const bool up = cm > m + 5.0f;
+      if (__any(up)) {
+        const float mn = up ? cm : m;
+        const float alpha = m == mn ? 1.0f : __builtin_amdgcn_exp2f(m - mn);   // exp2(-inf) = 0
+        lsum *= alpha;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) o[d] *= alpha;
+        m = mn;
+      }
+      const float ref = (m == ninf ? 0.0f : m) - 10.0f;   // p comes out times 2^10
+      float p[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        p[j] = __builtin_amdgcn_exp2f(fmaf(s[j], sc2, -ref));
+        lsum += p[j];
+      }
+      h8 ph[2], pl[2];
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2) {
+        u32x4 uh, ul;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float e0 = p[8 * s2 + 2 * k], e1 = p[8 * s2 + 2 * k + 1];
+          const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(e0, e1));
+          uh[k] = hi;
+          ul[k] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(fmaf(half_lo(hi), -1.0f, e0), fmaf(half_hi(hi), -1.0f, e1)));
+        }
+        ph[s2] = __builtin_bit_cast(h8, uh);
+        pl[s2] = __builtin_bit_cast(h8, ul);
+      }
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const int row = 32 * d + r;
+          const h8 vf = *reinterpret_cast<const h8*>(cV + vt_off<NK>(row, 4 * kv + 2 * s2 + h));
+          o[d] = mfma32(vf, ph[s2], o[d]);
+          o[d] = mfma32(vf, pl[s2], o[d]);
+        }
+      if (masked(kt)) {
+        uint32_t bad = s_bad[buf][kv];
+        while (bad) {                                     // workgroup-uniform, hardly ever entered
+          const int pos = __builtin_ctz(bad);             // of this wave's 32
+          bad &= bad - 1;
+          const int jj = 4 * (pos >> 3) + (pos & 3), hh = (pos >> 2) & 1;
+          float pv = 0.0f;
+#pragma unroll
+          for (int j = 0; j < 16; ++j) pv = j == jj ? p[j] : pv;
+          pv = __shfl(pv, r + 32 * hh);
+          const uint16_t* v = a.v_cache + head + (size_t)(p0 + pos) * kHeadDim;
+#pragma unroll
+          for (int d = 0; d < 4; ++d)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+              const uint16_t x = v[32 * d + 8 * (j >> 2) + 4 * h + (j & 3)];
+              if (p0 + pos < lim && f16_nonfinite(x)) o[d][j] = fmaf(pv, half_bits_to_float(x), o[d][j]);
+            }
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (more) store_v(kt + 1, buf ^ 1, nV);
+  };
+#pragma unroll 1
+  for (int kt = 0; kt < n_kt; kt += 2) {
+    tile(kt, 0, sK0, sV0, sK1, sV1);
+    if (kt + 1 < n_kt) tile(kt + 1, 1, sK1, sV1, sK0, sV0);
+  }
+  lsum += __shfl_xor(lsum, 32);                           // of the wave's positions
+  __syncthreads();                                        // the tiles are no longer read
+  // wave (qs, kv) finishes dims kOut kv .. of its rows: every wave leaves its
+  // sums of each wave's dims in that wave's buffer (a wave with no position
+  // has m = -inf)
+  constexpr int kD = 4 / NK, kOut = 32 * kD;   // 32-dim tiles, dims per finishing wave
+  float* xch[4] = {reinterpret_cast<float*>(sK0), reinterpret_cast<float*>(sK1), reinterpret_cast<float*>(sV0),
+                   reinterpret_cast<float*>(sV1)};        // by dim tile: [qs][source kv][16 values][64 lanes]
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) xch[d][((qs * NK + kv) * 16 + j) * 64 + l] = o[d][j];
+  if (h == 0) {
+    s_m[w][r] = m;
+    s_l[w][r] = lsum;
+  }
+  __syncthreads();
+  float M = ninf, L = 0.0f, e[NK];
+#pragma unroll
+  for (int k = 0; k < NK; ++k) M = fmaxf(M, s_m[qs + 2 * k][r]);
+#pragma unroll
+  for (int k = 0; k < NK; ++k) {
+    const float mk = s_m[qs + 2 * k][r];
+    e[k] = mk == ninf ? 0.0f : __builtin_amdgcn_exp2f(mk - M);
+    L = fmaf(e[k], s_l[qs + 2 * k][r], L);
+  }
+  const float inv = 1.0f / L;
+  if (tq < a.seq) {
+    uint16_t* po = a.out + ((size_t)bt * a.seq + tq) * kH + hq * kHeadDim + kOut * kv;
+#pragma unroll
+    for (int dd = 0; dd < kD; ++dd) {
+      const int d = kD * kv + dd;
+      const float* mine = reinterpret_cast<const float*>(d < 2 ? (d ? sK1 : sK0) : (d == 2 ? sV0 : sV1));
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int j = 4 * q4 + i;
+          v[i] = 0.0f;
+#pragma unroll
+          for (int k = 0; k < NK; ++k) v[i] = fmaf(e[k], mine[((qs * NK + k) * 16 + j) * 64 + l], v[i]);
+          v[i] *= inv;
+        }
+        *reinterpret_cast<u32x2v*>(po + 32 * dd + 8 * q4 + 4 * h) =
+            u32x2v{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])};
+      }
+    }
+  }
+}
+
 }  // namespace
 
 // The tile: the smallest whose tiles fit one workgroup per CU (64 rows, else
@@ -330,6 +623,18 @@ void launch_proj(const ProjArgs& a, int n_heads, hipStream_t st) {
     hipLaunchKernelGGL((k_proj<2, 128>), dim3(n8 * mt2), dim3(256), 0, st, a, mt2, n_heads);
   else
     hipLaunchKernelGGL((k_proj<2, 64>), dim3(n8 * mt2), dim3(256), 0, st, a, mt2, n_heads);
+}
+
+// Four position parts (eight waves, 128 positions a tile) while every
+// workgroup has a CU to itself, else two (two workgroups a CU): 1300 rows, 672
+// workgroups, 38.5 against 54.3 us; 9 rows over 4000 positions, 32 workgroups,
+// the layer 90 against 110 us.
+void launch_flash(const FlashArgs& a, hipStream_t st) {
+  const int n_qt = (a.seq + kFQ - 1) / kFQ, wgs = kH / kHeadDim * n_qt * a.batch;
+  if (wgs <= device_cus())
+    hipLaunchKernelGGL(k_flash<4>, dim3(wgs), dim3(512), 0, st, a, n_qt);
+  else
+    hipLaunchKernelGGL(k_flash<2>, dim3(wgs), dim3(256), 0, st, a, n_qt);
 }
 
 }  // namespace oi2

@@ -236,3 +236,38 @@ def test_prompt_rows_on_the_matrix_cores(dev, B, T, n_kv):
     x = torch.randn((B, T, H), generator=torch.Generator(device=dev).manual_seed(52), device=dev).half()
     cache = _rand_cache(dev, B, n_kv, past, seed=53) if past else None
     _check_step(attn, w, n_kv, x, cos[past:], sin[past:], cache, f"prompt B={B} T={T} n_kv={n_kv}")
+
+
+@pytest.mark.parametrize("B,T,past,n_kv", [(1, 9, 70, 8), (2, 64, 64, 32), (1, 65, 1023, 8), (2, 33, 4000, 4),
+                                           (1, 128, 0, 16), (1, 1100, 0, 8)])
+def test_prompt_attention_on_the_matrix_cores(dev, B, T, past, n_kv):
+    """Query rows at the edges of the prompt attention's 64-row tiles against
+    spans at the edges of its 64-position ones: chunks over a cache (every row
+    sees every position) and causal prompts, query groups of 1, 2, 4 and 8,
+    several sequences."""
+    w = _weights(dev, n_kv, seed=61 + T)
+    attn = oi2.GroupedQueryAttention(0, w, _cfg(n_kv))
+    cos, sin = oi2.rope_tables(past + T, D, 1e6, device=dev)
+    x = torch.randn((B, T, H), generator=torch.Generator(device=dev).manual_seed(62), device=dev).half()
+    cache = _rand_cache(dev, B, n_kv, past, seed=63) if past else None
+    _check_step(attn, w, n_kv, x, cos[past:], sin[past:], cache, f"attention B={B} T={T} past={past} n_kv={n_kv}")
+
+
+@pytest.mark.parametrize("bad", [5, 40, 63, 64, 90])
+def test_a_prompt_row_does_not_see_later_non_finite_values(dev, bad):
+    """A position whose v overflows fp16 (and so is inf) spoils the rows that
+    see it and no earlier row, wherever it lies in a tile of positions: the
+    rows before it equal those of the prompt cut off before it."""
+    n_kv, T = 8, 100
+    w = _weights(dev, n_kv, seed=71)
+    w["layer_000.v_proj"] = torch.full((n_kv * D, H), 96.0, device=dev).to(torch.float8_e4m3fn)
+    w["layer_000.input_layernorm"] = torch.ones(H, dtype=torch.float16, device=dev)
+    cos, sin = oi2.rope_tables(T, D, 1e6, device=dev)
+    x = torch.randn((1, T, H), generator=torch.Generator(device=dev).manual_seed(72), device=dev).half()
+    x[0, bad] = 1.0                                        # v = 4096 * 96
+    out, (_, v) = oi2.GroupedQueryAttention(0, w, _cfg(n_kv))(x, cos, sin)
+    cut, _ = oi2.GroupedQueryAttention(0, w, _cfg(n_kv))(x[:, :bad].contiguous(), cos, sin)
+    assert torch.isinf(v[0, :, bad]).all() and torch.isfinite(v[0, :, :bad]).all()
+    assert torch.isfinite(out[0, :bad]).all()
+    assert_ffn_close(out[0, :bad].float().cpu().numpy(), cut[0].float().cpu().numpy(), tol=2e-3, what="rows before")
+    assert not torch.isfinite(out[0, bad:]).any()
