@@ -31,59 +31,103 @@ struct QuantArgs {
   uint8_t* records;           // record k at records + 6400 k
 };
 
-// One workgroup per (record k = blockIdx.x, vector m = blockIdx.y): thread t
-// quantises elements 16 t .. 16 t + 15, i.e. one eighth of group t / 8.
-__global__ __launch_bounds__(kThreads) void k_quantize_records(QuantArgs a) {
-  const int k = blockIdx.x, m = blockIdx.y, t = threadIdx.x;
-  const int64_t es = a.elem_stride[m];
-  const float* v = a.src[m] + (int64_t)a.rows[k] * a.row_stride[m] + (int64_t)(16 * t) * es;
-  float x[16];
-  if (es == 1 && (reinterpret_cast<uintptr_t>(v) & 15) == 0) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const f32x4 q = reinterpret_cast<const f32x4*>(v)[i];
-      x[4 * i] = q.x;
-      x[4 * i + 1] = q.y;
-      x[4 * i + 2] = q.z;
-      x[4 * i + 3] = q.w;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) x[i] = v[i * es];
-  }
-  float amax = 0.0f;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(x[i]));
-  // the 8 threads of a group are consecutive lanes
-  amax = fmaxf(amax, __shfl_xor(amax, 1, kWave));
-  amax = fmaxf(amax, __shfl_xor(amax, 2, kWave));
-  amax = fmaxf(amax, __shfl_xor(amax, 4, kWave));
-  const float s = __fdiv_rn(fmaxf(amax, 1e-8f), 7.0f);
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
+// q = clamp(rint(x / s), -8, 7) as 4 bits, the quotient correctly rounded
+// first.  inv = 1 / s gives x / s to within 3 ulp (1.5e-6 at |x / s| <= 7),
+// which rounds to the same integer unless it lies that close to a tie; only
+// then is the division made (a correctly rounded one is ~10 instructions).
+// NaN and infinite operands behave in x inv as in x / s.
+__device__ __forceinline__ uint32_t quant4(float x, float s, float inv) {
+  float d = x * inv;
+  float r = __builtin_rintf(d);
+  if (__builtin_expect(fabsf(fabsf(d - r) - 0.5f) < 4e-6f, 0)) r = __builtin_rintf(__fdiv_rn(x, s));
+  return (uint32_t)(int)fminf(fmaxf(r, -8.0f), 7.0f) & 0xFu;
+}
+
+__device__ __forceinline__ float group_scale(float amax) { return __fdiv_rn(fmaxf(amax, 1e-8f), 7.0f); }
+
+// A vector whose elements are consecutive (gate and up rows): one workgroup
+// per (record k, vector m).  Thread t takes elements
+// 4 t .. 4 t + 3 of each 1024, so a wave's load is 1 KB in one piece and a
+// group is half a wave.  (16 consecutive elements a thread made every load
+// touch 64 pieces 64 bytes apart.)
+__device__ __forceinline__ void quantize_row(const QuantArgs& a, int k, int m) {
+  const int t = threadIdx.x;
+  const float* v = a.src[m] + (int64_t)a.rows[k] * a.row_stride[m];
+  f32x4 x[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) x[c] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_a4*>(v + 1024 * c + 4 * t));
   uint8_t* rec = a.records + (size_t)k * kRecBytes;
-  uint16_t* out = reinterpret_cast<uint16_t*>(rec + kOffGate + m * (kH / 2) + 8 * t);   // 2-byte aligned
+  uint16_t* out = reinterpret_cast<uint16_t*>(rec + kOffGate + m * (kH / 2)) + t;
 #pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    uint32_t half = 0;
+  for (int c = 0; c < 4; ++c) {
+    float amax = fmaxf(fmaxf(fabsf(x[c].x), fabsf(x[c].y)), fmaxf(fabsf(x[c].z), fabsf(x[c].w)));
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float r = __builtin_rintf(__fdiv_rn(x[4 * p + j], s));
-      const int q = (int)fminf(fmaxf(r, -8.0f), 7.0f);
-      half |= (uint32_t)(q & 0xF) << (4 * j);
-    }
-    out[p] = (uint16_t)half;
+    for (int o = 1; o < 32; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, kWave));
+    const float s = group_scale(amax), inv = __fdiv_rn(1.0f, s);
+    out[256 * c] = (uint16_t)(quant4(x[c].x, s, inv) | (quant4(x[c].y, s, inv) << 4) | (quant4(x[c].z, s, inv) << 8) |
+                              (quant4(x[c].w, s, inv) << 12));
+    if ((t & 31) == 0)
+      reinterpret_cast<uint16_t*>(rec + kOffScales + m * kGroups * 2)[8 * c + (t >> 5)] = float_to_half_bits(s);
   }
-  if ((t & 7) == 0)
-    reinterpret_cast<uint16_t*>(rec + kOffScales + m * kGroups * 2)[t >> 3] = float_to_half_bits(s);
   if (m == 0) {
     if (t == 0) reinterpret_cast<uint16_t*>(rec)[0] = a.nids[k];
     if (t < (kRecBytes - kRawRecord) / 2) reinterpret_cast<uint16_t*>(rec + kRawRecord)[t] = 0;
   }
 }
 
+// Vectors whose elements are strided (the down matrix's columns): lanes are
+// records, so that a load of one element reads neighbouring columns of one
+// matrix row.  Workgroup: 64 records x kColGroups groups of 128 elements, wave
+// w elements 32 w .. 32 w + 31 of each group; the next group's loads are in
+// flight while one is quantised.  Neighbouring record tiles share the lines
+// at their edges and run on one XCD.  (A workgroup per record and vector read
+// 4 bytes of every line of the columns: a 10752-record section took 696 us.)
+constexpr int kColGroups = 4;
+__device__ __forceinline__ void quantize_cols(const QuantArgs& a, int tile, int m, int g0,
+                                              float (&s_max)[2][4][kWave]) {
+  const int l = lane_id(), w = threadIdx.x >> 6;
+  const int k = tile * kWave + l, kc = k < a.n ? k : a.n - 1;
+  const int64_t es = a.elem_stride[m];
+  const float* v = a.src[m] + (int64_t)a.rows[kc] * a.row_stride[m] + (int64_t)(kGroup * g0 + 32 * w) * es;
+  uint8_t* rec = a.records + (size_t)kc * kRecBytes;
+  float x[2][32];
+  auto load = [&](int g, float (&d)[32]) {
+    const float* p = v + (int64_t)(kGroup * g) * es;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) d[i] = p[i * es];
+  };
+  load(0, x[0]);
+#pragma unroll
+  for (int g = 0; g < kColGroups; ++g) {
+    const int cur = g & 1;
+    if (g + 1 < kColGroups) load(g + 1, x[cur ^ 1]);
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(x[cur][i]));
+    s_max[cur][w][l] = amax;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // the next loads stay in flight
+    amax = fmaxf(fmaxf(s_max[cur][0][l], s_max[cur][1][l]), fmaxf(s_max[cur][2][l], s_max[cur][3][l]));
+    const float s = group_scale(amax), inv = __fdiv_rn(1.0f, s);
+    u32x4 q = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 32; ++i) q[i >> 3] |= quant4(x[cur][i], s, inv) << (4 * (i & 7));
+    if (k < a.n) {
+      *reinterpret_cast<u32x4_a2*>(rec + kOffGate + m * (kH / 2) + (g0 + g) * (kGroup / 2) + 16 * w) = q;
+      if (w == 0)
+        reinterpret_cast<uint16_t*>(rec + kOffScales + m * kGroups * 2)[g0 + g] = float_to_half_bits(s);
+    }
+  }
+  if (m == 0 && g0 == 0 && w == 0 && k < a.n) {
+    reinterpret_cast<uint16_t*>(rec)[0] = a.nids[k];
+    for (int i = 0; i < (kRecBytes - kRawRecord) / 2; ++i) reinterpret_cast<uint16_t*>(rec + kRawRecord)[i] = 0;
+  }
+}
+
 // Header and trailing zero padding of a section with n records.
-__global__ __launch_bounds__(kThreads) void k_section_frame(uint8_t* section, int layer, int expert, int n,
-                                                            size_t body, size_t total) {
+__device__ __forceinline__ void section_frame(uint8_t* section, int layer, int expert, int n, size_t body,
+                                              size_t total) {
   const int t = threadIdx.x;
   if (t == 0) {
     uint32_t* h = reinterpret_cast<uint32_t*>(section);
@@ -93,6 +137,41 @@ __global__ __launch_bounds__(kThreads) void k_section_frame(uint8_t* section, in
     h[3] = 0;
   }
   for (size_t i = body + t; i < total; i += kThreads) section[i] = 0;
+}
+
+// One launch: workgroup 0 frames the section, the next take the strided
+// vectors (8 per tiles x kGroups / kColGroups each; the longest ones first),
+// the rest one consecutive vector each.  Bound by memory: a 10752-record
+// section reads 528 MB and writes 69 MB in 139 us, 4.3 TB/s (a large copy
+// moves 4.8); in launches of their own 75 + 77 + 4 us, and 145 with the rows'
+// loads not marked non-temporal.
+struct SectionArgs {
+  QuantArgs q;
+  int rows_v[3], cols_v[3], n_rows, n_cols;   // vectors by kind
+  int tiles, per;                             // 64-record tiles, and per XCD
+  uint8_t* section;
+  int layer, expert;
+  size_t body, total;
+};
+__global__ __launch_bounds__(kThreads) void k_quantize_section(SectionArgs a) {
+  __shared__ float s_max[2][4][kWave];
+  int b = blockIdx.x;
+  if (b == 0) {
+    section_frame(a.section, a.layer, a.expert, a.q.n, a.body, a.total);
+    return;
+  }
+  b -= 1;
+  constexpr int kParts = kGroups / kColGroups;
+  const int x8 = 8 * a.per, cols = a.n_cols * kParts * x8;
+  if (b < cols) {
+    const int v = b / (kParts * x8), r = b - v * kParts * x8, part = r / x8, t = r - part * x8;
+    // XCD t & 7 takes a run of tiles: neighbours share the lines at their edges
+    const int tile = (t & 7) * a.per + (t >> 3);
+    if (tile < a.tiles) quantize_cols(a.q, tile, a.cols_v[v], part * kColGroups, s_max);
+    return;
+  }
+  b -= cols;
+  quantize_row(a.q, b % a.q.n, a.rows_v[b / a.q.n]);
 }
 
 size_t section_bytes(int64_t n) {
@@ -121,6 +200,12 @@ extern "C" int oi2_quantize_section(int32_t layer, int32_t expert, int32_t n, co
   OI2_CHECK_ARG(section_bytes_ >= need, "section buffer of %zu bytes is smaller than the %zu required",
                 section_bytes_, need);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  SectionArgs sa{};
+  sa.section = section;
+  sa.layer = layer;
+  sa.expert = expert;
+  sa.body = (size_t)kHeader + (size_t)n * kRecBytes;
+  sa.total = need;
   if (n > 0) {
     OI2_CHECK_ARG(nids && rows && gate && up && down && row_stride && elem_stride,
                   "nids, rows, gate, up, down and the strides are required");
@@ -137,11 +222,16 @@ extern "C" int oi2_quantize_section(int32_t layer, int32_t expert, int32_t n, co
     a.rows = rows;
     a.n = n;
     a.records = section + kHeader;
-    hipLaunchKernelGGL(k_quantize_records, dim3(n, 3), dim3(kThreads), 0, st, a);
-    OI2_CHECK_LAUNCH();
+    for (int m = 0; m < 3; ++m) {
+      if (elem_stride[m] == 1) sa.rows_v[sa.n_rows++] = m;
+      else sa.cols_v[sa.n_cols++] = m;
+    }
+    sa.q = a;
   }
-  hipLaunchKernelGGL(k_section_frame, dim3(1), dim3(kThreads), 0, st, section, layer, expert, n,
-                     (size_t)kHeader + (size_t)n * kRecBytes, need);
+  sa.tiles = (n + kWave - 1) / kWave;
+  sa.per = (sa.tiles + 7) / 8;
+  const int64_t grid = 1 + (int64_t)sa.n_cols * (kGroups / kColGroups) * 8 * sa.per + (int64_t)sa.n_rows * n;
+  hipLaunchKernelGGL(k_quantize_section, dim3((unsigned)grid), dim3(kThreads), 0, st, sa);
   OI2_CHECK_LAUNCH();
   return OI2_OK;
 }

@@ -107,3 +107,24 @@ def test_device_writer_empty_section(dev):
     z = torch.zeros((0, H), dtype=torch.float32, device=dev)
     sec = quantize_section_rows(7, z, z, z, [])
     assert sec.cpu().numpy().tobytes() == fmt.section_bytes(7, np.zeros((0, fmt.NEURON_RECORD_BYTES), np.uint8))
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 130])
+def test_strided_vectors_match_the_host_writer(dev, n):
+    """All three vectors read as columns (element stride > 1), in no order of
+    ids, at the edges of the 64-record tiles; column 0 is made of ties, whose
+    quotients decide between two integers."""
+    from oi2.split import _run
+    rng = np.random.default_rng(n)
+    width = 200
+    mats = [(rng.standard_normal((H, width)) * 0.02).astype(np.float32) for _ in range(3)]
+    rows = rng.permutation(width)[:n]
+    ties = (rng.integers(-14, 15, H) / 2).astype(np.float32)
+    ties.reshape(-1, 128)[:, 0] = 7.0                       # scale 1 in every group
+    for m, mat in enumerate(mats):
+        mat[:, rows[0]] = ties * np.float32(3.0 ** m)       # and 3, 9: quotients at the ties, inexact reciprocals
+    t = [torch.as_tensor(m, device=dev) for m in mats]
+    nids = np.arange(500, 500 + n)
+    sec = _run(3, 0, *t, torch.as_tensor(rows, device=dev), nids, (1, 1, 1), (width, width, width)).cpu().numpy()
+    ref = fmt.section_bytes(3, fmt.build_records(nids, *[m.T[rows] for m in mats]))
+    assert sec.tobytes() == ref
