@@ -848,7 +848,8 @@ __global__ __launch_bounds__(kThreads) void k_pgemm_down_hot(BDownArgs a, int mt
 // the whole range sit in an LDS table, so no load waits for another.
 constexpr int kDcItems = 64;                // items per K block
 constexpr int kLdC = kDcItems + 8;          // LDS row of T and of the H tile, halves (144 B)
-constexpr int kDcMaxItems = 2048;           // items per workgroup (record offset table)
+constexpr int kDcMaxItems = 2048;           // items per workgroup of the separate cold down (record offset table)
+constexpr int kDcTab = 32;                  // joint down: K blocks per half of its record offset table
 
 // 8 x 8 nibble transpose: r[k] nibble n -> r[n] nibble k.
 __device__ __forceinline__ void nibble_transpose8(uint32_t (&r)[8]) {
@@ -1103,7 +1104,7 @@ __global__ __launch_bounds__(2 * kThreads) void k_pgemm_down_both(BDownArgs a, i
   constexpr int kColdT = 256 * kLdC * 2, kColdH = 32 * MS * kLdC * 2;
   constexpr int kBuf = kHotA + kHotB > kColdT + kColdH ? kHotA + kHotB : kColdT + kColdH;
   __shared__ __attribute__((aligned(16))) uint8_t smem[2 * kBuf];
-  __shared__ uint32_t s_rec[kDcMaxItems];
+  __shared__ uint32_t s_rec[2 * kDcTab * kDcItems];   // record offsets of the range's blocks, two halves in turn
   __shared__ __attribute__((aligned(16))) uint16_t s_sc[4 * kDcItems];
   const int b = blockIdx.x;
   const int q = b >> 3, per = mt * splits;
@@ -1123,11 +1124,17 @@ __global__ __launch_bounds__(2 * kThreads) void k_pgemm_down_both(BDownArgs a, i
     // of outputs j0 + 8 (t >> 3) of items 8 (t & 7) .. + 7, and chunk t & 7
     // of H_cold rows (t >> 3) + 32 r
     const int t = threadIdx.x - 256, wp = w - 4;
-    for (int i = t; i < nc * kDcItems; i += kThreads) {
-      const int it = cb0 * kDcItems + i;
-      const int slot = it < total ? a.dslots[it] : -1;
-      s_rec[i] = (slot >= 0 && slot < a.n_records) ? (uint32_t)slot * kRecBytes : kNoOffset;
-    }
+    // record offsets of the range's blocks c0 .. c0 + kDcTab - 1 into their
+    // half of the table
+    auto fill = [&](int c0) {
+      for (int i = t; i < min(nc - c0, kDcTab) * kDcItems; i += kThreads) {
+        const int it = (cb0 + c0) * kDcItems + i;
+        const int slot = it < total ? a.dslots[it] : -1;
+        s_rec[(c0 % (2 * kDcTab)) * kDcItems + i] =
+            (slot >= 0 && slot < a.n_records) ? (uint32_t)slot * kRecBytes : kNoOffset;
+      }
+    };
+    fill(0);
     const rsrc_t rha = buf_rsrc(a.hh, (uint32_t)a.M * a.ldh * 2);
     const rsrc_t rd = buf_rsrc(a.down_q, (uint32_t)kH * a.down_stride);
     const rsrc_t rr = buf_rsrc(a.records, (uint32_t)a.n_records * kRecBytes);
@@ -1156,7 +1163,7 @@ __global__ __launch_bounds__(2 * kThreads) void k_pgemm_down_both(BDownArgs a, i
         for (int r = 0; r < 8; ++r) R[sl][2 * MS + r] = bload16(rd, doff[r], kb * kBK);
       } else {
         const int kb = cb0 + i - nh;
-        const int ib = (i - nh) * kDcItems;
+        const int ib = (i - nh) % (2 * kDcTab) * kDcItems;
 #pragma unroll
         for (int k = 0; k < 8; ++k)
           R[sl][k >> 2][k & 3] = __builtin_amdgcn_raw_buffer_load_b32(rr, (int)(s_rec[ib + 8 * ig + k] + dbyte), 0, 0);
@@ -1248,6 +1255,9 @@ __global__ __launch_bounds__(2 * kThreads) void k_pgemm_down_both(BDownArgs a, i
             __builtin_amdgcn_sched_barrier(0);
             if (i + 3 < n) load(i + 3, u ^ 1);
           }
+          // the next half of the table, a barrier before its first use
+          const int c = i + 3 - nh;
+          if (c >= 0 && c % kDcTab == kDcTab - 2 && c + 2 < nc) fill(c + 2);
           lds_barrier();
         }
       }
@@ -1862,17 +1872,16 @@ __global__ __launch_bounds__(kThreads) void k_bfinal16(const float* part, int n_
 }
 
 // Dense copy of a chunked active list (any chunk size): dslots[0 .. total).
+// One workgroup per chunk, each with the whole prefix (56 chunks of 256 one
+// after the other in one workgroup took 30 us).
 __global__ __launch_bounds__(kThreads) void k_bcompact(ActiveList al, int cap, int32_t* dslots,
                                                       int32_t* total) {
   __shared__ int s_prefix[kMaxChunks + 1];
   chunk_prefix(al, s_prefix);
-  for (int c = 0; c < al.n_chunks; ++c) {
-    const int base = s_prefix[c];
-    const int cnt = s_prefix[c + 1] - base;
-    for (int k = threadIdx.x; k < cnt; k += kThreads)
-      if (base + k < cap) dslots[base + k] = al.slots[(size_t)c * al.chunk + k];
-  }
-  if (threadIdx.x == 0) *total = min(s_prefix[al.n_chunks], cap);
+  const int c = blockIdx.x, base = s_prefix[c], cnt = s_prefix[c + 1] - base;
+  for (int k = threadIdx.x; k < cnt; k += kThreads)
+    if (base + k < cap) dslots[base + k] = al.slots[(size_t)c * al.chunk + k];
+  if (c == 0 && threadIdx.x == 0) *total = min(s_prefix[al.n_chunks], cap);
 }
 
 // ── host ────────────────────────────────────────────────────────────────────
@@ -1946,10 +1955,12 @@ static BatchPlan batch_plan(int M, int n_hot, int cap) {
   // (separate hot and cold downs, or the ranges of the joint one)
   p.both_splits = 0;
   if (M > kSkinnyMax && n_hot > 0 && cap > 0) {
-    if (p.pms == 4)
-      p.both_splits = std::max(p.hot_splits, cold_down_splits(M, cap));
-    else
-      p.both_splits = std::max(cold_down_splits(M, cap), std::min(p.hot_blocks, 256 / (16 * p.pmt)));
+    // about 256 workgroups, whatever the list's capacity: a drop-in layer's
+    // list has room for every neuron, and one range per 2048 of it made a
+    // 1300-token prompt with 540 active records write and add seven partial
+    // sums (down 84 us, final add 26; one range: 70 and 9)
+    const int n_blk = (cap + kDcItems - 1) / kDcItems, want = std::max(1, 256 / (16 * p.pmt));
+    p.both_splits = std::max(std::min(p.hot_blocks, want), std::min(n_blk, want));
   }
   const int y_parts = M <= kSkinnyMax ? 1
                                       : std::max(p.both_splits, (n_hot > 0 ? p.hot_splits : 0) +
@@ -2034,7 +2045,7 @@ int batch_ffn(const uint16_t* x, int M, const uint16_t* norm_w, float eps, const
     dtotal = active->counts;
   } else if (has_cold) {
     ActiveList al{active->slots, active->counts, active->n_chunks, active->chunk};
-    hipLaunchKernelGGL(k_bcompact, dim3(1), dim3(kThreads), 0, st, al, cap, dslots, total);
+    hipLaunchKernelGGL(k_bcompact, dim3(active->n_chunks), dim3(kThreads), 0, st, al, cap, dslots, total);
     OI2_CHECK_LAUNCH();
   }
   BUpArgs ua{};
