@@ -645,3 +645,31 @@ def test_sparse_ffn_layer_file_residency(dev, direct_io):
             ex.shutdown()
             fstore.close()
             hstore.close()
+
+
+@pytest.mark.parametrize("rows,n_hot,n_cold,hot_dt,cold_dt", [
+    (1, 1, 33, torch.float16, torch.float32), (2, 15, 0, torch.bfloat16, torch.float32), (3, 7, 8, torch.float16, torch.bfloat16),
+    (13, 100, 17, torch.float16, torch.float32), (16, 0, 31, torch.float16, torch.bfloat16),
+    (17, 64, 65, torch.float32, torch.float16), (64, 255, 96, torch.float16, torch.float32),
+    (65, 48, 16, torch.bfloat16, torch.bfloat16), (130, 33, 7, torch.float32, torch.float32)])
+def test_sparse_ffn_tensors_at_tile_edges(dev, rows, n_hot, n_cold, hot_dt, cold_dt):
+    """sparse_ffn on dense tensors at the edges of its 16-token, 16-neuron and
+    32-neuron pieces and of its 64-token passes, every weight type in either
+    half, against float64 over the same tensors.  The result is fp16 of fp32
+    sums of up to 4096 + 255 terms: half an fp16 ulp (2^-11 relative) and a
+    few 1e-6 of the sums' size."""
+    g = torch.Generator(device=dev).manual_seed(rows)
+    x = torch.randn((rows, H), generator=g, device=dev).half()
+
+    def half(n, dt):
+        return [(torch.randn(s, generator=g, device=dev) * 0.02).to(dt) for s in ((n, H), (n, H), (H, n))]
+    hot, cold = half(n_hot, hot_dt), half(n_cold, cold_dt)
+    for act, both in (("silu", False), ("relu", True)):
+        y = oi2.sparse_ffn(x, act, both, *hot, *cold).double()
+        f = torch.relu if act == "relu" else lambda v: v * torch.sigmoid(v)
+        ref = torch.zeros((rows, H), dtype=torch.float64, device=dev)
+        for G, U, D in (hot, cold):
+            a, u = x.double() @ G.double().t(), x.double() @ U.double().t()
+            ref += (f(a) * (f(u) if both else u)) @ D.double().t()
+        err = (y - ref).abs() - ref.abs() * 2.0 ** -11
+        assert float(err.max()) <= 1e-5 * float(ref.abs().max()) + 2.0 ** -25, (act, float(err.max()))
