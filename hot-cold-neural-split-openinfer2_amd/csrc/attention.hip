@@ -36,11 +36,12 @@ namespace {
 
 constexpr int kHd = kHeadDim;
 constexpr int kHalf = kHd / 2;
-constexpr int kMaxRows = 8;              // token rows per GEMV launch
-// From these rows on the projections run on the matrix cores (attn_prompt.hip):
-// the GEMV takes 17.2 + 8.2 us per 8 rows (q / k / v and o_proj), k_rmsnorm and
-// k_proj 3 + 18 + 16 us from 9 rows to 64.
-constexpr int kPromptRows = 9;
+constexpr int kMaxRows = 8;              // token rows per GEMV launch (of those past kPromptMaxRows)
+// From these rows on the projections run on the matrix cores (attn_prompt.hip),
+// behind a norm launch of their own.  A whole layer at 200 cached positions,
+// GEMV against these: 4 rows 22.2, 23.9 us; 5 rows 24.5, 24.3; 6 rows 27.2,
+// 24.9; 8 rows 31.7, 26.9; 16 rows (two GEMV passes) 57.8, 32.5.
+constexpr int kPromptRows = 6;
 constexpr int kFlashSeq = 9;             // rows of a sequence from which attention runs on the matrix cores
 constexpr int kFlashMaxSpan = 1 << 23;   // 32-bit byte offsets into one head's cache
 constexpr int kPromptMaxRows = 0x7FFFFFFF / (kH * 2);   // 32-bit byte offsets into the rows
@@ -852,12 +853,10 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
     p.seq = seq;
     p.cos = cos;
     p.sin = sin;
+    p.counters = counters;
+    p.n_counters = past + seq > kOneWgMax && !flash ? rows * n_kv : 0;
     launch_proj(p, n_q + 2 * n_kv, st);
     OI2_CHECK_LAUNCH();
-    if (past + seq > kOneWgMax && !flash) {
-      hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(kThreads), 0, st, counters, rows * n_kv, 0u);
-      OI2_CHECK_LAUNCH();
-    }
   }
   for (int r0 = 0; !prompt && r0 < rows; r0 += kMaxRows) {
     const int rc = rows - r0 < kMaxRows ? rows - r0 : kMaxRows;

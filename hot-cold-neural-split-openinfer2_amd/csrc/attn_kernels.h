@@ -26,6 +26,8 @@ struct ProjArgs {
   int n_kv, cap, past, seq;
   const float* cos;           // (seq, 64)
   const float* sin;
+  uint32_t* counters;         // n_counters words that the launch clears
+  int n_counters;
   // mode 1
   uint16_t* out;              // (rows, H)
   const uint16_t* residual;   // (rows, H) or null

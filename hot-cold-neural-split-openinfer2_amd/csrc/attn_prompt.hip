@@ -105,6 +105,8 @@ __global__ __launch_bounds__(256, KB == 64 ? 2 : 1) void k_proj(ProjArgs a, int 
   __shared__ __align__(1024) uint8_t sB0[kPB], sB1[kPB], sB2[kPB];
   const int b = blockIdx.x, q = b >> 3;
   const int hb = (q / mt) * 8 + (b & 7);
+  if (b == 0)
+    for (int i = threadIdx.x; i < a.n_counters; i += 256) a.counters[i] = 0u;
   if (hb >= n_heads) return;                   // the whole workgroup
   const int m0 = (q % mt) * kBM;
   const int l = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -308,6 +310,114 @@ __global__ __launch_bounds__(256, KB == 64 ? 2 : 1) void k_proj(ProjArgs a, int 
     }
     *reinterpret_cast<u32x4*>(dst) = v0;
     *reinterpret_cast<u32x4*>(dst + kHalfHead) = v1;
+  }
+}
+
+// ── projections of a few rows ────────────────────────────────────────────────
+//
+// At most 16 NT rows: bound by the weight stream.  Workgroup: 16 weight rows
+// of a head, the eight RoPE pairs (j, j + 64) from j0 on as columns 0-7 and
+// 8-15 of one 16x16x32 MFMA, its eight waves 512 K each; the waves' sums meet
+// in LDS.  Lane l = (t, q) = (l % 16, l / 16) takes 16 bytes (16 K, two steps)
+// of weight row t and the same 16 K of token t straight from memory: nothing
+// is shared between the waves, so nothing goes through LDS before the sums.
+// 8 rows: q / k / v 11.0 us (the single-token GEMV 18.2), o_proj 7.5 (9.6);
+// a layer at 12 rows 30 us (k_proj's 64-row tiles: 46), at 32 rows 48 (53),
+// and at 48 rows, four token tiles, 67 (61).
+constexpr int kFewThreads = 512, kFewWaves = 8;
+
+template <int NT>
+__global__ __launch_bounds__(kFewThreads, 4) void k_proj_few(ProjArgs a) {
+  __shared__ f32x4 s_r[kFewWaves][kWave];
+  const int l = lane_id(), t = l & 15, q = l >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hb = blockIdx.x >> 3, j0 = 8 * (blockIdx.x & 7);
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < a.n_counters; i += kFewThreads) a.counters[i] = 0u;
+  const uint8_t* W;
+  int blk;
+  if (hb < a.blocks0) {
+    W = a.w0;
+    blk = hb;
+  } else if (hb < a.blocks0 + a.blocks1) {
+    W = a.w1;
+    blk = hb - a.blocks0;
+  } else {
+    W = a.w2;
+    blk = hb - a.blocks0 - a.blocks1;
+  }
+  const uint8_t* pw = W + (size_t)(blk * kHeadDim + j0 + (t & 7) + kHalfHead * (t >> 3)) * kH + 512 * w + 16 * q;
+  const rsrc_t rx = rsrc(a.x, (uint32_t)a.rows * kH * 2);      // rows past the call read zero
+  const uint32_t x0 = ((uint32_t)t * kH + 512 * w + 16 * q) * 2;
+  f32x4 acc[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  constexpr int kB = NT == 1 ? 8 : 4;                          // 64-wide K chunks loaded together
+#pragma unroll 1
+  for (int c0 = 0; c0 < 8; c0 += kB) {
+    u32x4 wv[kB], xv[kB][NT][2];
+#pragma unroll
+    for (int c = 0; c < kB; ++c) {
+      wv[c] = load16_nt(pw + 64 * (c0 + c));
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+          xv[c][nt][s] = bld16(rx, x0 + nt * (16 * kH * 2) + 128 * (c0 + c) + 16 * s);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < kB; ++c)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const h8 b = fp8x8_h8(wv[c][2 * s], wv[c][2 * s + 1]);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, xv[c][nt][s]), b, acc[nt], 0, 0, 0);
+      }
+  }
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    if (nt > 0) __syncthreads();                               // the previous sums are read
+    s_r[w][l] = acc[nt];
+    __syncthreads();
+    // thread i < 128: row i / 8, pair i % 8
+    const int r = threadIdx.x >> 3, p = threadIdx.x & 7, row = 16 * nt + r, j = j0 + p;
+    if (r >= 16 || row >= a.rows) continue;
+    float y0 = 0.0f, y1 = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kFewWaves; ++k) {
+      y0 += s_r[k][16 * (r >> 2) + p][r & 3];
+      y1 += s_r[k][16 * (r >> 2) + 8 + p][r & 3];
+    }
+    y0 = round_f16(y0);
+    y1 = round_f16(y1);
+    if (a.mode == 1) {
+      const size_t o = (size_t)row * kH + hb * kHeadDim + j;
+      a.out[o] = float_to_half_bits(y0);
+      a.out[o + kHalfHead] = float_to_half_bits(y1);
+      if (a.residual) {
+        a.x_out[o] = float_to_half_bits(half_bits_to_float(a.residual[o]) + y0);
+        a.x_out[o + kHalfHead] = float_to_half_bits(half_bits_to_float(a.residual[o + kHalfHead]) + y1);
+      }
+      continue;
+    }
+    const int bt = row / a.seq, tt = row - bt * a.seq;
+    float o0 = y0, o1 = y1;
+    if (hb < a.blocks0 + a.blocks1) {
+      const float c = round_f16(a.cos[(size_t)tt * kHalfHead + j]), s = round_f16(a.sin[(size_t)tt * kHalfHead + j]);
+      o0 = y0 * c - y1 * s;
+      o1 = y0 * s + y1 * c;
+    }
+    uint16_t* dst;
+    if (hb < a.blocks0) {
+      dst = a.q + (size_t)row * a.q_width + blk * kHeadDim + j;
+    } else {
+      uint16_t* cache = hb < a.blocks0 + a.blocks1 ? a.k_cache : a.v_cache;
+      dst = cache + (((size_t)bt * a.n_kv + blk) * a.cap + (a.past + tt)) * kHeadDim + j;
+    }
+    dst[0] = float_to_half_bits(o0);
+    dst[kHalfHead] = float_to_half_bits(o1);
   }
 }
 
@@ -604,7 +714,8 @@ __global__ __launch_bounds__(128 * NK, 4 / NK) void k_flash(FlashArgs a, int n_q
 
 }  // namespace
 
-// The tile: the smallest whose tiles fit one workgroup per CU (64 rows, else
+// Up to 32 rows (16 with 96 heads, whose 768 workgroups of two token tiles take
+// longer: a layer at 32 rows 105 against 92 us) k_proj_few.  From there the smallest tile whose tiles fit one workgroup per CU (64 rows, else
 // 128 rows, on 128-wide K blocks: three deep buffers of one workgroup fill a
 // CU's LDS); past that 128 rows on 64-wide K blocks, two workgroups a CU.
 // Measured, q / k / v (48 heads) and o_proj (32 heads) in us:
@@ -615,6 +726,11 @@ __global__ __launch_bounds__(128 * NK, 4 / NK) void k_flash(FlashArgs a, int n_q
 //   768    55.5  37.4    58.7  31.5    49.6  31.8
 //   1000   66.7  43.1    64.0  34.6    57.7  37.2
 void launch_proj(const ProjArgs& a, int n_heads, hipStream_t st) {
+  if (a.rows <= 16 || (a.rows <= 32 && n_heads <= 64)) {
+    if (a.rows <= 16) hipLaunchKernelGGL(k_proj_few<1>, dim3(8 * n_heads), dim3(kFewThreads), 0, st, a);
+    else hipLaunchKernelGGL(k_proj_few<2>, dim3(8 * n_heads), dim3(kFewThreads), 0, st, a);
+    return;
+  }
   const int cus = device_cus();
   const int mt1 = (a.rows + 63) / 64, mt2 = (a.rows + 127) / 128, n8 = (n_heads + 7) / 8 * 8;
   if (mt1 * n_heads <= cus)

@@ -223,9 +223,11 @@ def test_rewind_decodes_a_position_again_in_place(dev):
 
 
 @pytest.mark.parametrize("B,T,n_kv", [(1, 9, 8), (1, 63, 32), (1, 64, 8), (2, 65, 4), (1, 129, 8), (3, 43, 16),
-                                      (1, 400, 8), (1, 700, 32), (11, 1, 8)])
+                                      (1, 400, 8), (1, 700, 32), (11, 1, 8), (6, 1, 4), (1, 16, 32), (1, 17, 8),
+                                      (2, 16, 16), (1, 33, 8), (1, 17, 32)])
 def test_prompt_rows_on_the_matrix_cores(dev, B, T, n_kv):
-    """Rows at the edges of the prompt projections' 64- and 128-row tiles and
+    """Rows at the edges of the projections' kernels for a few rows (6 to 16, 17
+    to 32), of the prompt projections' 64- and 128-row tiles and
     of their choice of tile (400 rows with 48 heads and 700 rows with 96 fill
     more than one tile per CU), several sequences with rows of each in one
     tile, a batch of single rows over a cache."""
