@@ -151,7 +151,9 @@ def load_library():
 def lib():
     """The library, for compute calls: also requires a visible GPU."""
     L = load_library()
-    if not torch.cuda.is_available():
+    # an initialised runtime has a GPU; asking it for its devices on every call
+    # costs several microseconds
+    if not torch.cuda.is_initialized() and not torch.cuda.is_available():
         raise OI2Error("oi2 kernels need a gfx950 GPU; none is visible")
     return L
 
@@ -177,8 +179,17 @@ def dtype_code(dtype) -> int:
 
 
 def stream_handle(device=None) -> int | None:
-    s = torch.cuda.current_stream(device).cuda_stream
-    return s or None
+    """The current stream of a device (the current device by default) as the
+    C ABI takes it; read as a raw handle, a tenth of the cost of building a
+    torch.cuda.Stream."""
+    index = device.index if isinstance(device, torch.device) else device
+    if index is None:
+        index = torch.cuda.current_device()
+    elif not isinstance(index, int):
+        return torch.cuda.current_stream(device).cuda_stream or None
+    else:
+        torch.cuda.init()
+    return torch._C._cuda_getCurrentRawStream(index) or None
 
 
 def logit_threshold(p: float) -> float:

@@ -20,6 +20,7 @@ import torch
 
 from . import _lib
 from .format import HIDDEN_DIM
+from .store import host_ids, to_device
 
 
 def section_nbytes(n_cold: int) -> int:
@@ -46,8 +47,8 @@ def quantize_section(layer: int, gate: torch.Tensor, up: torch.Tensor, down: tor
     inter, hidden = gate.shape
     if hidden != HIDDEN_DIM or up.shape != gate.shape or down.shape != (hidden, inter):
         raise ValueError(f"expected gate/up ({inter}, {HIDDEN_DIM}) and down ({HIDDEN_DIM}, {inter})")
-    rows = torch.as_tensor(np.asarray(list(cold_ids), np.int64), device=dev)
-    if rows.numel() and (int(rows.min()) < 0 or int(rows.max()) >= inter):
+    rows = host_ids(cold_ids)
+    if rows.size and (int(rows.min()) < 0 or int(rows.max()) >= inter):
         raise ValueError("cold ids out of range")
     return _run(layer, expert, gate, up, down, rows, nids if nids is not None else rows,
                 (hidden, hidden, 1), (1, 1, inter))
@@ -65,28 +66,30 @@ def quantize_section_rows(layer: int, gate: torch.Tensor, up: torch.Tensor, down
         if t.dim() != 2 or t.shape[1] != HIDDEN_DIM or t.shape[0] != gate.shape[0]:
             raise ValueError(f"{name} must be (n, {HIDDEN_DIM})")
     n = gate.shape[0]
-    rows = torch.arange(n, device=dev, dtype=torch.int64)
+    rows = np.arange(n, dtype=np.int64)
     return _run(layer, expert, gate, up, down_cols, rows, nids,
                 (HIDDEN_DIM, HIDDEN_DIM, HIDDEN_DIM), (1, 1, 1))
 
 
 def _run(layer, expert, gate, up, down, rows, nids, row_stride, elem_stride):
+    """rows and nids are host ids; both go to the device in one copy."""
     L = _lib.lib()
     dev = gate.device
-    n = int(rows.numel())
-    ids = np.asarray(torch.as_tensor(nids).cpu().numpy() if torch.is_tensor(nids) else list(nids),
-                     np.int64).reshape(-1)
+    n = int(rows.size)
+    ids = rows if nids is rows else host_ids(nids)
     if ids.size != n:
         raise ValueError("one id per record is required")
     if n and (ids.min() < 0 or ids.max() > 0xFFFF):
         raise ValueError("neuron ids must fit the record's u16 id field")
-    nid16 = torch.as_tensor(ids.astype(np.uint16).view(np.int16), device=dev)
-    rows32 = rows.to(torch.int32)
+    packed = np.empty(2 * n + (n + 1) // 2 * 2, dtype=np.int16)     # rows as int32, then nids as u16
+    packed[:2 * n].view(np.int32)[:] = rows
+    packed[2 * n:3 * n] = ids.astype(np.uint16).view(np.int16)
+    packed = to_device(packed, dev)
     size = int(L.oi2_section_bytes(n))
     out = torch.empty(size, dtype=torch.uint8, device=dev)
     rs = (ctypes.c_int64 * 3)(*row_stride)
     es = (ctypes.c_int64 * 3)(*elem_stride)
-    _lib.check(L.oi2_quantize_section(int(layer), int(expert), n, _lib.ptr(nid16), _lib.ptr(rows32),
+    _lib.check(L.oi2_quantize_section(int(layer), int(expert), n, packed.data_ptr() + 4 * n, packed.data_ptr(),
                                       _lib.ptr(gate), _lib.ptr(up), _lib.ptr(down),
                                       ctypes.cast(rs, ctypes.c_void_p), ctypes.cast(es, ctypes.c_void_p),
                                       _lib.ptr(out), size, _lib.stream_handle(dev)))

@@ -15,6 +15,7 @@ three arguments the store returns CPU tensors, as splitter.py:397-403 does;
 """
 from __future__ import annotations
 
+import array
 import mmap
 import threading
 
@@ -23,6 +24,37 @@ import torch
 
 from . import _lib
 from . import format as fmt
+
+
+def host_ids(ids) -> np.ndarray:
+    """Neuron ids (any iterable of integers, or an array) as flat int64.  A list
+    of ints goes through array.array, two thirds of the time of numpy's own
+    conversion; whatever that does not take (floats, nested sequences) goes
+    through numpy."""
+    if isinstance(ids, np.ndarray):
+        return ids.astype(np.int64, copy=False).reshape(-1)
+    if torch.is_tensor(ids):
+        return ids.cpu().numpy().astype(np.int64, copy=False).reshape(-1)
+    ids = ids if isinstance(ids, list) else list(ids)
+    if not ids:
+        return np.zeros(0, dtype=np.int64)
+    try:
+        return np.frombuffer(array.array("q", ids), dtype=np.int64)
+    except (TypeError, OverflowError):
+        return np.asarray(ids, dtype=np.int64).reshape(-1)
+
+
+def to_device(a: np.ndarray, device) -> torch.Tensor:
+    """A host array on the device, in stream order: through pinned memory of
+    torch's caching host allocator, so that the call does not wait for the
+    copy (a pageable copy does).  Under stream capture it is a pageable copy,
+    which the capture refuses: a recorded copy would read the pinned memory
+    again at every replay."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.from_numpy(a).to(device)
+    t = torch.empty(a.shape, dtype=torch.from_numpy(a[:0]).dtype, pin_memory=True)
+    t.numpy()[...] = a
+    return t.to(device, non_blocking=True)
 
 
 class ColdSection:
@@ -46,8 +78,10 @@ class ColdSection:
 
     def slots_for(self, neuron_ids) -> np.ndarray:
         """Request-order slots of the ids present in the section."""
-        ids = np.asarray(list(neuron_ids) if not isinstance(neuron_ids, np.ndarray) else neuron_ids,
-                         dtype=np.int64).reshape(-1)
+        ids = host_ids(neuron_ids)
+        if ids.size and ids.min() >= 0 and ids.max() < self.inter:
+            slots = self.lut_host[ids]
+            return slots if slots.min() >= 0 else slots[slots >= 0]
         ok = (ids >= 0) & (ids < self.inter)
         slots = np.full(ids.shape, -1, dtype=np.int32)
         slots[ok] = self.lut_host[ids[ok]]
@@ -213,7 +247,7 @@ class ColdWeightStore:
         gate = torch.empty((n, self.H), dtype=torch.float32, device=dev)
         up = torch.empty((n, self.H), dtype=torch.float32, device=dev)
         down = torch.empty((self.H, n), dtype=torch.float32, device=dev)
-        s = torch.as_tensor(slots).to(dev)
+        s = to_device(slots, dev)
         _lib.check(L.oi2_dequant_records(sec.records.data_ptr(), sec.n_records, s.data_ptr(), n,
                                          gate.data_ptr(), up.data_ptr(), down.data_ptr(),
                                          _lib.stream_handle(dev)))

@@ -125,6 +125,6 @@ def test_strided_vectors_match_the_host_writer(dev, n):
         mat[:, rows[0]] = ties * np.float32(3.0 ** m)       # and 3, 9: quotients at the ties, inexact reciprocals
     t = [torch.as_tensor(m, device=dev) for m in mats]
     nids = np.arange(500, 500 + n)
-    sec = _run(3, 0, *t, torch.as_tensor(rows, device=dev), nids, (1, 1, 1), (width, width, width)).cpu().numpy()
+    sec = _run(3, 0, *t, rows.astype(np.int64), nids, (1, 1, 1), (width, width, width)).cpu().numpy()
     ref = fmt.section_bytes(3, fmt.build_records(nids, *[m.T[rows] for m in mats]))
     assert sec.tobytes() == ref

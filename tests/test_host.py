@@ -240,3 +240,15 @@ def test_file_store_direct_read_gap(gap):
                     _lib.check(_lib.load_library().oi2_file_store_set_read_gap(fs._h, bad))
         finally:
             fs.close()
+
+
+def test_host_ids_takes_what_numpy_took():
+    """Neuron ids in every form the calls accept come out as numpy's own
+    conversion of the list gave them."""
+    from oi2.store import host_ids
+    for ids in ([], [5], [3, 3, -1, 70000], range(7), (1, 2), [np.int32(4), 9], [1.9, -2.2], [[1, 2], [3, 4]],
+                np.array([[7, 8]], np.int32), np.array([1.5, 2.5]), torch.tensor([4, 2], dtype=torch.int32)):
+        want = np.asarray(ids if isinstance(ids, np.ndarray) else [int(v) for v in ids] if torch.is_tensor(ids)
+                          else list(ids), dtype=np.int64).reshape(-1)
+        got = host_ids(ids)
+        assert got.dtype == np.int64 and np.array_equal(got, want), ids
