@@ -79,6 +79,7 @@ struct SdpaArgs {
   const uint16_t* k_cache;
   const uint16_t* v_cache;
   int n_kv, cap, past, seq, causal, n_split, part_stride;
+  int chunks;                 // chunks per wave of the looping k_attn_sdpa; 0: the one-shot one
   float scale;
   float* part;                // (rows, n_kv, n_split, part_stride)
   uint32_t* counters;         // (rows, n_kv)
@@ -305,7 +306,20 @@ __global__ __launch_bounds__(kThreads) void k_attn_gemv(GemvArgs a) {
 // partials of (r, g) merges them into the fp16 output, its loads all
 // independent of each other (the m / l table first, then 16-byte pieces of
 // the partial sums, several in flight per thread).
-template <int G, int STEPS>
+//
+// LOOP: a.chunks (even) such spans per workgroup, the next one's loads in
+// flight under each one's products, with a running max per 16-lane position
+// group.  The one-shot form loads everything, then computes everything, and
+// its reductions over lanes, waves and splits follow every 128 positions; once
+// there are 256 workgroups of 256 positions each, half as many of them hide
+// more (whole layer, one-shot and LOOP, us: n_kv 8, 8 sequences at 2000
+// positions 42.5 and 39.8, 2 at 4000 30.8 and 28.7, 1 at 8000 32.0 and 28.2;
+// n_kv 16, 4 at 2000 37.0 and 34.8; n_kv 32, 1 at 4000 35.7 and 31.4).  512
+// positions per workgroup: 43.2, 32.4, 31.0, 35.3, 30.8.  With 8 query heads
+// per kv head its registers leave one wave per SIMD and it is slower (8 at
+// 3000: 51.0 and 55.4).
+constexpr int kLoopSteps = 4, kLoopChunks = 4;
+template <int G, int STEPS, bool LOOP>
 __global__ __launch_bounds__(kThreads) void k_attn_sdpa(SdpaArgs a) {
   extern __shared__ float s_tab[];                 // merge: m then l, (n_split, G) each
   // the waves' partial sums; later the merge's per-group sums (1024 floats)
@@ -320,87 +334,136 @@ __global__ __launch_bounds__(kThreads) void k_attn_sdpa(SdpaArgs a) {
   const int b = r / a.seq, t = r - b * a.seq;
   const int n_r = a.causal ? a.past + t + 1 : a.past + a.seq;
   const int width = a.n_kv * G * kHd;
-  const int base = split * 4 * kPW + wave * kPW;
+  const int n_chunk = LOOP ? a.chunks : 1;
+  const int base = split * n_chunk * 4 * kPW + wave * kPW;
 
   u32x4 qv[G];
 #pragma unroll
   for (int h = 0; h < G; ++h)
     qv[h] = *reinterpret_cast<const u32x4*>(a.q + (size_t)r * width + (g * G + h) * kHd + 8 * jj);
   const size_t head = ((size_t)b * a.n_kv + g) * a.cap;
-  u32x4 kr[STEPS], vr[STEPS];
+  struct Rows {
+    u32x4 k[STEPS], v[STEPS];
+  };
+  // chunk c: positions base + 4 kPW c + 4 it + k, those past n_r clamped
+  auto load = [&](int c, Rows& x) {
+    const int p0 = base + 4 * kPW * c + k;
 #pragma unroll
-  for (int it = 0; it < STEPS; ++it) {
-    const int p = base + 4 * it + k;
-    const int pc = p < n_r ? p : n_r - 1;
-    kr[it] = *reinterpret_cast<const u32x4*>(a.k_cache + (head + pc) * kHd + 8 * jj);
-  }
-#pragma unroll
-  for (int it = 0; it < STEPS; ++it) {
-    const int p = base + 4 * it + k;
-    const int pc = p < n_r ? p : n_r - 1;
-    vr[it] = *reinterpret_cast<const u32x4*>(a.v_cache + (head + pc) * kHd + 8 * jj);
-  }
-
-  float s[STEPS * G];
-#pragma unroll
-  for (int it = 0; it < STEPS; ++it)
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      float d = 0.0f;
-#pragma unroll
-      for (int m = 0; m < 4; ++m) d = dot2(as_f16x2(kr[it][m]), as_f16x2(qv[h][m]), d);
-      s[it * G + h] = d;
+    for (int it = 0; it < STEPS; ++it) {
+      const int p = p0 + 4 * it;
+      const int pc = p < n_r ? p : n_r - 1;
+      x.k[it] = *reinterpret_cast<const u32x4*>(a.k_cache + (head + pc) * kHd + 8 * jj);
     }
-  // sums over the 16 lanes of each row: every lane of the row gets the total
 #pragma unroll
-  for (int e = 0; e < STEPS * G; ++e) s[e] += dpp_f<0xB1>(s[e]);
-#pragma unroll
-  for (int e = 0; e < STEPS * G; ++e) s[e] += dpp_f<0x4E>(s[e]);
-#pragma unroll
-  for (int e = 0; e < STEPS * G; ++e) s[e] += dpp_f<0x141>(s[e]);
-#pragma unroll
-  for (int e = 0; e < STEPS * G; ++e) s[e] += dpp_f<0x140>(s[e]);
+    for (int it = 0; it < STEPS; ++it) {
+      const int p = p0 + 4 * it;
+      const int pc = p < n_r ? p : n_r - 1;
+      x.v[it] = *reinterpret_cast<const u32x4*>(a.v_cache + (head + pc) * kHd + 8 * jj);
+    }
+  };
 
   const float ninf = -__builtin_inff();
-  float mx[G];
-#pragma unroll
-  for (int h = 0; h < G; ++h) mx[h] = ninf;
-#pragma unroll
-  for (int it = 0; it < STEPS; ++it) {
-    const bool ok = base + 4 * it + k < n_r;
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      s[it * G + h] = ok ? s[it * G + h] * a.scale : ninf;
-      mx[h] = fmaxf(mx[h], s[it * G + h]);
-    }
-  }
+  float mx[G], l[G], o[G][8];
 #pragma unroll
   for (int h = 0; h < G; ++h) {
-    mx[h] = fmaxf(mx[h], __shfl_xor(mx[h], 16));
-    mx[h] = fmaxf(mx[h], __shfl_xor(mx[h], 32));
-  }
-  float l[G], o[G][8];
-#pragma unroll
-  for (int h = 0; h < G; ++h) {
+    mx[h] = ninf;
     l[h] = 0.0f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[h][e] = 0.0f;
   }
+  auto use = [&](int c, const Rows& x) {
+    const int p0 = base + 4 * kPW * c + k;
+    float s[STEPS * G];
 #pragma unroll
-  for (int it = 0; it < STEPS; ++it) {
-    float vf[8];
+    for (int it = 0; it < STEPS; ++it)
 #pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      vf[2 * d] = half_lo(vr[it][d]);
-      vf[2 * d + 1] = half_hi(vr[it][d]);
+      for (int h = 0; h < G; ++h) {
+        float d = 0.0f;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) d = dot2(as_f16x2(x.k[it][m]), as_f16x2(qv[h][m]), d);
+        s[it * G + h] = d;
+      }
+    // sums over the 16 lanes of each row: every lane of the row gets the total
+#pragma unroll
+    for (int e = 0; e < STEPS * G; ++e) s[e] += dpp_f<0xB1>(s[e]);
+#pragma unroll
+    for (int e = 0; e < STEPS * G; ++e) s[e] += dpp_f<0x4E>(s[e]);
+#pragma unroll
+    for (int e = 0; e < STEPS * G; ++e) s[e] += dpp_f<0x141>(s[e]);
+#pragma unroll
+    for (int e = 0; e < STEPS * G; ++e) s[e] += dpp_f<0x140>(s[e]);
+    float mo[G];
+#pragma unroll
+    for (int h = 0; h < G; ++h) mo[h] = mx[h];
+#pragma unroll
+    for (int it = 0; it < STEPS; ++it) {
+      const bool ok = p0 + 4 * it < n_r;
+#pragma unroll
+      for (int h = 0; h < G; ++h) {
+        s[it * G + h] = ok ? s[it * G + h] * a.scale : ninf;
+        mx[h] = fmaxf(mx[h], s[it * G + h]);
+      }
     }
 #pragma unroll
     for (int h = 0; h < G; ++h) {
-      const float sv = s[it * G + h];
-      const float p = sv == ninf ? 0.0f : __expf(sv - mx[h]);
-      l[h] += p;
+      if (LOOP) {
+        // the sums so far at the new max (zero while there is none)
+        const float sc = mo[h] == ninf ? 0.0f : __expf(mo[h] - mx[h]);
+        l[h] *= sc;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[h][e] = fmaf(p, vf[e], o[h][e]);
+        for (int e = 0; e < 8; ++e) o[h][e] *= sc;
+      } else {
+        mx[h] = fmaxf(mx[h], __shfl_xor(mx[h], 16));
+        mx[h] = fmaxf(mx[h], __shfl_xor(mx[h], 32));
+      }
+    }
+#pragma unroll
+    for (int it = 0; it < STEPS; ++it) {
+      float vf[8];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        vf[2 * d] = half_lo(x.v[it][d]);
+        vf[2 * d + 1] = half_hi(x.v[it][d]);
+      }
+#pragma unroll
+      for (int h = 0; h < G; ++h) {
+        const float sv = s[it * G + h];
+        const float p = sv == ninf ? 0.0f : __expf(sv - mx[h]);
+        l[h] += p;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[h][e] = fmaf(p, vf[e], o[h][e]);
+      }
+    }
+  };
+  if (!LOOP) {
+    Rows x;
+    load(0, x);
+    use(0, x);
+  } else {
+    // an even number of chunks, the next one's loads in flight under each
+    Rows x0, x1;
+    load(0, x0);
+    int c = 0;
+#pragma unroll 1
+    for (; c + 2 < n_chunk; c += 2) {
+      load(c + 1, x1);
+      use(c, x0);
+      load(c + 2, x0);
+      use(c + 1, x1);
+    }
+    load(c + 1, x1);
+    use(c, x0);
+    use(c + 1, x1);
+    // the four position groups' sums at the wave's max
+#pragma unroll
+    for (int h = 0; h < G; ++h) {
+      const float m = mx[h];
+      mx[h] = fmaxf(mx[h], __shfl_xor(mx[h], 16));
+      mx[h] = fmaxf(mx[h], __shfl_xor(mx[h], 32));
+      const float sc = m == ninf ? 0.0f : __expf(m - mx[h]);
+      l[h] *= sc;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[h][e] *= sc;
     }
   }
 #pragma unroll
@@ -700,10 +763,16 @@ void launch_gemv(const GemvArgs& a, int rows, int blocks, hipStream_t st) {
 template <int G>
 void launch_sdpa_g(const SdpaArgs& a, int steps, int rows, size_t lds, hipStream_t st) {
   const dim3 grid(a.n_split, a.n_kv, rows);
+  if constexpr (G <= 4) {
+    if (a.chunks > 0) {
+      hipLaunchKernelGGL((k_attn_sdpa<G, kLoopSteps, true>), grid, dim3(kThreads), lds, st, a);
+      return;
+    }
+  }
   switch (steps) {
-    case 2: hipLaunchKernelGGL((k_attn_sdpa<G, 2>), grid, dim3(kThreads), lds, st, a); break;
-    case 4: hipLaunchKernelGGL((k_attn_sdpa<G, 4>), grid, dim3(kThreads), lds, st, a); break;
-    default: hipLaunchKernelGGL((k_attn_sdpa<G, 8>), grid, dim3(kThreads), lds, st, a); break;
+    case 2: hipLaunchKernelGGL((k_attn_sdpa<G, 2, false>), grid, dim3(kThreads), lds, st, a); break;
+    case 4: hipLaunchKernelGGL((k_attn_sdpa<G, 4, false>), grid, dim3(kThreads), lds, st, a); break;
+    default: hipLaunchKernelGGL((k_attn_sdpa<G, 8, false>), grid, dim3(kThreads), lds, st, a); break;
   }
 }
 
@@ -735,9 +804,9 @@ struct WsLayout {
   size_t q, attn, counters, part, total;
 };
 
-// The split partial sums are sized for the launch the call makes: none when
-// the span (past + seq positions) fits one workgroup per query head, else
-// the splits choose_steps picks for that span.
+// The split partial sums: none when the span (past + seq positions) fits one
+// workgroup per query head, else the splits choose_steps picks for that span
+// (the looping kernel makes at most as many).
 WsLayout ws_layout(int rows, int n_q, int n_kv, int span) {
   const int G = n_q / n_kv;
   const int per_split = span <= kOneWgMax ? 0 : 16 * choose_steps(rows, n_kv, span);
@@ -902,11 +971,17 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
     const int steps = choose_steps(rows, n_kv, past + seq);
     s.n_split = (past + seq + 16 * steps - 1) / (16 * steps);
     s.part_stride = part_stride_floats(G);
-    const size_t tab = (size_t)2 * s.n_split * G * sizeof(float);
+    size_t tab = (size_t)2 * s.n_split * G * sizeof(float);
     if (tab > (size_t)kMaxTabBytes) {
       set_error("%d positions need %d sequence splits; the merge table holds %d", past + seq, s.n_split,
                 kMaxTabBytes / (int)(2 * G * sizeof(float)));
       return OI2_EUNSUPPORTED;
+    }
+    const int per = 16 * kLoopSteps * kLoopChunks, n_loop = (past + seq + per - 1) / per;
+    if (G <= 4 && (int64_t)rows * n_kv * n_loop >= 256) {   // fewer, longer splits: the workspace holds them
+      s.chunks = kLoopChunks;
+      s.n_split = n_loop;
+      tab = (size_t)2 * n_loop * G * sizeof(float);
     }
     s.part = part;
     s.counters = counters;

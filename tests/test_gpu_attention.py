@@ -105,6 +105,23 @@ def test_decode_step_against_oracle(dev, B, past, n_kv):
     _check_step(attn, w, n_kv, x, cos[past:], sin[past:], cache, f"decode B={B} past={past} n_kv={n_kv}")
 
 
+@pytest.mark.parametrize("B,T,past,n_kv", [(8, 1, 1024, 8), (1, 1, 8191, 8), (1, 1, 8192, 8), (1, 1, 7935, 8),
+                                           (4, 1, 1280, 16), (2, 1, 1055, 32), (1, 5, 2040, 8), (8, 1, 2100, 4)])
+def test_long_spans_in_looping_splits(dev, B, T, past, n_kv):
+    """Spans whose 256-position splits number at least 256: the last split of
+    one position, of all 256 and of most of them, one split fewer (one-shot
+    splits) and 8 query heads per kv head (always one-shot); keys that grow
+    along the span, so every chunk raises the running max."""
+    w = _weights(dev, n_kv, seed=past + n_kv)
+    attn = oi2.GroupedQueryAttention(0, w, _cfg(n_kv))
+    cos, sin = oi2.rope_tables(past + T, D, 10000.0, device=dev)
+    g = torch.Generator(device=dev).manual_seed(11)
+    x = torch.randn((B, T, H), generator=g, device=dev).half()
+    k, v = _rand_cache(dev, B, n_kv, past, seed=past)
+    k *= torch.linspace(0.1, 2.0, past, device=dev).half()[:, None]
+    _check_step(attn, w, n_kv, x, cos[past:], sin[past:], (k, v), f"B={B} T={T} past={past} n_kv={n_kv}")
+
+
 def test_prefill_then_decode_like_the_engine(dev):
     """engine.py:406-442's use: a causal prefill without a cache, then
     decode steps that pass back the cache the previous call returned (the
