@@ -1,8 +1,9 @@
 // Grouped-query attention for decode on gfx950: GroupedQueryAttention.forward
 // (engine.py:90-125) with the KV cache kept in place.
 //
-// One call runs three kernels on its stream (with 9 and more token rows k_proj
-// and, for rows enough, k_flash of attn_prompt.hip, k_rmsnorm ahead of them):
+// One call runs three kernels on its stream (from 6 token rows the projections
+// are attn_prompt.hip's, behind a norm launch, and with rows enough per
+// sequence so is the attention):
 //   k_attn_gemv (qkv)  RMSNorm of the token rows (input_layernorm,
 //                      engine.py:93), then q, k, v = fp16(x_n W^T) from the
 //                      fp8 e4m3fn weights (the reference keeps them fp8 at
@@ -311,14 +312,19 @@ __global__ __launch_bounds__(kThreads) void k_attn_gemv(GemvArgs a) {
 // flight under each one's products, with a running max per 16-lane position
 // group.  The one-shot form loads everything, then computes everything, and
 // its reductions over lanes, waves and splits follow every 128 positions; once
-// there are 256 workgroups of 256 positions each, half as many of them hide
+// workgroups of 256 positions nearly fill the chip, half as many of them hide
 // more (whole layer, one-shot and LOOP, us: n_kv 8, 8 sequences at 2000
 // positions 42.5 and 39.8, 2 at 4000 30.8 and 28.7, 1 at 8000 32.0 and 28.2;
 // n_kv 16, 4 at 2000 37.0 and 34.8; n_kv 32, 1 at 4000 35.7 and 31.4).  512
-// positions per workgroup: 43.2, 32.4, 31.0, 35.3, 30.8.  With 8 query heads
-// per kv head its registers leave one wave per SIMD and it is slower (8 at
-// 3000: 51.0 and 55.4).
-constexpr int kLoopSteps = 4, kLoopChunks = 4;
+// positions per workgroup: 43.2, 32.4, 31.0, 35.3, 30.8.  8 query heads per
+// kv head take chunks of half the length (n_kv 4: 16 sequences at 2000 59.5
+// and 51.8, 8 at 3000 51.3 and 48.7; with the others' chunks, 55.4).
+constexpr int kLoopSpan = 256;           // positions per workgroup
+// 216 workgroups (n_kv 8, one sequence at 6900 positions) 30.5 one-shot, 27.6;
+// 224 (n_kv 16, 2 at 1700) 26.7, 25.6; 192 (n_kv 8, 3 at 2000) 27.9, 28.2; 168
+// (3 at 1700) 27.7, 28.3.
+constexpr int kLoopMinWgs = 208;
+constexpr int loop_steps(int G) { return G == 8 ? 2 : 4; }
 template <int G, int STEPS, bool LOOP>
 __global__ __launch_bounds__(kThreads) void k_attn_sdpa(SdpaArgs a) {
   extern __shared__ float s_tab[];                 // merge: m then l, (n_split, G) each
@@ -763,11 +769,9 @@ void launch_gemv(const GemvArgs& a, int rows, int blocks, hipStream_t st) {
 template <int G>
 void launch_sdpa_g(const SdpaArgs& a, int steps, int rows, size_t lds, hipStream_t st) {
   const dim3 grid(a.n_split, a.n_kv, rows);
-  if constexpr (G <= 4) {
-    if (a.chunks > 0) {
-      hipLaunchKernelGGL((k_attn_sdpa<G, kLoopSteps, true>), grid, dim3(kThreads), lds, st, a);
-      return;
-    }
+  if (a.chunks > 0) {
+    hipLaunchKernelGGL((k_attn_sdpa<G, loop_steps(G), true>), grid, dim3(kThreads), lds, st, a);
+    return;
   }
   switch (steps) {
     case 2: hipLaunchKernelGGL((k_attn_sdpa<G, 2, false>), grid, dim3(kThreads), lds, st, a); break;
@@ -864,6 +868,14 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
   const WsLayout L = ws_layout(rows, n_q, n_kv, past + seq);
   OI2_CHECK_ARG(workspace && workspace_bytes >= L.total, "workspace of %zu bytes, %zu needed",
                 workspace_bytes, L.total);
+  // spans past the merge table are refused whichever kernels would run
+  const int steps = choose_steps(rows, n_kv, past + seq);
+  const int n_split = past + seq > kOneWgMax ? (past + seq + 16 * steps - 1) / (16 * steps) : 1;
+  if ((size_t)2 * n_split * G * sizeof(float) > (size_t)kMaxTabBytes) {
+    set_error("%d positions need %d sequence splits; the merge table holds %d", past + seq, n_split,
+              kMaxTabBytes / (int)(2 * G * sizeof(float)));
+    return OI2_EUNSUPPORTED;
+  }
   hipStream_t st = (hipStream_t)stream;
   uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
   uint16_t* qb = reinterpret_cast<uint16_t*>(ws + L.q);
@@ -968,21 +980,14 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
     launch_sdpa1(s, G, rows, st);
     OI2_CHECK_LAUNCH();
   } else {
-    const int steps = choose_steps(rows, n_kv, past + seq);
-    s.n_split = (past + seq + 16 * steps - 1) / (16 * steps);
+    s.n_split = n_split;
     s.part_stride = part_stride_floats(G);
-    size_t tab = (size_t)2 * s.n_split * G * sizeof(float);
-    if (tab > (size_t)kMaxTabBytes) {
-      set_error("%d positions need %d sequence splits; the merge table holds %d", past + seq, s.n_split,
-                kMaxTabBytes / (int)(2 * G * sizeof(float)));
-      return OI2_EUNSUPPORTED;
-    }
-    const int per = 16 * kLoopSteps * kLoopChunks, n_loop = (past + seq + per - 1) / per;
-    if (G <= 4 && (int64_t)rows * n_kv * n_loop >= 256) {   // fewer, longer splits: the workspace holds them
-      s.chunks = kLoopChunks;
+    const int n_loop = (past + seq + kLoopSpan - 1) / kLoopSpan;
+    if ((int64_t)rows * n_kv * n_loop >= kLoopMinWgs) {   // fewer, longer splits: the workspace holds them
+      s.chunks = kLoopSpan / (16 * loop_steps(G));
       s.n_split = n_loop;
-      tab = (size_t)2 * n_loop * G * sizeof(float);
     }
+    const size_t tab = (size_t)2 * s.n_split * G * sizeof(float);
     s.part = part;
     s.counters = counters;
     launch_sdpa(s, G, steps, rows, tab, st);

@@ -105,13 +105,14 @@ def test_decode_step_against_oracle(dev, B, past, n_kv):
     _check_step(attn, w, n_kv, x, cos[past:], sin[past:], cache, f"decode B={B} past={past} n_kv={n_kv}")
 
 
-@pytest.mark.parametrize("B,T,past,n_kv", [(8, 1, 1024, 8), (1, 1, 8191, 8), (1, 1, 8192, 8), (1, 1, 7935, 8),
-                                           (4, 1, 1280, 16), (2, 1, 1055, 32), (1, 5, 2040, 8), (8, 1, 2100, 4)])
+@pytest.mark.parametrize("B,T,past,n_kv", [(8, 1, 1024, 8), (1, 1, 8191, 8), (1, 1, 8192, 8), (1, 1, 6400, 8),
+                                           (1, 1, 6399, 8), (4, 1, 1280, 16), (2, 1, 1055, 32), (1, 5, 2040, 8),
+                                           (8, 1, 2100, 4), (7, 1, 1792, 4), (7, 1, 1791, 4)])
 def test_long_spans_in_looping_splits(dev, B, T, past, n_kv):
-    """Spans whose 256-position splits number at least 256: the last split of
+    """Spans whose 256-position splits number at least 208: the last split of
     one position, of all 256 and of most of them, one split fewer (one-shot
-    splits) and 8 query heads per kv head (always one-shot); keys that grow
-    along the span, so every chunk raises the running max."""
+    splits), query groups of 1, 2, 4 and 8; keys that grow along the span, so
+    every chunk raises the running max."""
     w = _weights(dev, n_kv, seed=past + n_kv)
     attn = oi2.GroupedQueryAttention(0, w, _cfg(n_kv))
     cos, sin = oi2.rope_tables(past + T, D, 10000.0, device=dev)
