@@ -182,7 +182,11 @@ def stream_handle(device=None) -> int | None:
     """The current stream of a device (the current device by default) as the
     C ABI takes it; read as a raw handle, a tenth of the cost of building a
     torch.cuda.Stream."""
-    index = device.index if isinstance(device, torch.device) else device
+    if isinstance(device, torch.device):
+        if device.type != "cuda":
+            raise ValueError(f"expected a GPU device, got {device}")
+        device = device.index
+    index = device
     if index is None:
         index = torch.cuda.current_device()
     elif not isinstance(index, int):

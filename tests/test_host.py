@@ -252,3 +252,11 @@ def test_host_ids_takes_what_numpy_took():
                           else list(ids), dtype=np.int64).reshape(-1)
         got = host_ids(ids)
         assert got.dtype == np.int64 and np.array_equal(got, want), ids
+
+
+def test_stream_handle_refuses_a_host_device():
+    """A host tensor's device has no stream: a call on one stops here, before
+    its pointer reaches a kernel."""
+    for device in (torch.device("cpu"), torch.device("meta")):
+        with pytest.raises(ValueError):
+            _lib.stream_handle(device)
