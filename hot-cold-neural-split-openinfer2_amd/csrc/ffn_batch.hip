@@ -1097,14 +1097,16 @@ __global__ __launch_bounds__(kThreads) void k_pgemm_down_cold(BDownArgs a, int m
 // loaded two ahead and go through two LDS buffers, one barrier per block;
 // a buffer holds either kind.  (With 4 waves doing both, 512 tokens took
 // 4219 against 3958 us per 32 layers, 64 tokens 1868 against 1834.)
-template <int MS>
+// LONG: the range may have more blocks than the record offset table, whose
+// halves are then refilled in turn as the loop goes.
+template <int MS, bool LONG>
 __global__ __launch_bounds__(2 * kThreads) void k_pgemm_down_both(BDownArgs a, int mt, int splits) {
   constexpr int NB = 2;
   constexpr int kHotA = 32 * MS * kLdA * 2, kHotB = 256 * kLdB8;   // bytes per buffer
   constexpr int kColdT = 256 * kLdC * 2, kColdH = 32 * MS * kLdC * 2;
   constexpr int kBuf = kHotA + kHotB > kColdT + kColdH ? kHotA + kHotB : kColdT + kColdH;
   __shared__ __attribute__((aligned(16))) uint8_t smem[2 * kBuf];
-  __shared__ uint32_t s_rec[2 * kDcTab * kDcItems];   // record offsets of the range's blocks, two halves in turn
+  __shared__ uint32_t s_rec[2 * kDcTab * kDcItems];   // record offsets of the range's blocks
   __shared__ __attribute__((aligned(16))) uint16_t s_sc[4 * kDcItems];
   const int b = blockIdx.x;
   const int q = b >> 3, per = mt * splits;
@@ -1124,10 +1126,10 @@ __global__ __launch_bounds__(2 * kThreads) void k_pgemm_down_both(BDownArgs a, i
     // of outputs j0 + 8 (t >> 3) of items 8 (t & 7) .. + 7, and chunk t & 7
     // of H_cold rows (t >> 3) + 32 r
     const int t = threadIdx.x - 256, wp = w - 4;
-    // record offsets of the range's blocks c0 .. c0 + kDcTab - 1 into their
-    // half of the table
+    // record offsets of the range's blocks from c0 on: all of them, or half a
+    // table
     auto fill = [&](int c0) {
-      for (int i = t; i < min(nc - c0, kDcTab) * kDcItems; i += kThreads) {
+      for (int i = t; i < (LONG ? min(nc - c0, kDcTab) : nc) * kDcItems; i += kThreads) {
         const int it = (cb0 + c0) * kDcItems + i;
         const int slot = it < total ? a.dslots[it] : -1;
         s_rec[(c0 % (2 * kDcTab)) * kDcItems + i] =
@@ -1163,7 +1165,7 @@ __global__ __launch_bounds__(2 * kThreads) void k_pgemm_down_both(BDownArgs a, i
         for (int r = 0; r < 8; ++r) R[sl][2 * MS + r] = bload16(rd, doff[r], kb * kBK);
       } else {
         const int kb = cb0 + i - nh;
-        const int ib = (i - nh) % (2 * kDcTab) * kDcItems;
+        const int ib = (LONG ? (i - nh) % (2 * kDcTab) : i - nh) * kDcItems;
 #pragma unroll
         for (int k = 0; k < 8; ++k)
           R[sl][k >> 2][k & 3] = __builtin_amdgcn_raw_buffer_load_b32(rr, (int)(s_rec[ib + 8 * ig + k] + dbyte), 0, 0);
@@ -1255,9 +1257,10 @@ __global__ __launch_bounds__(2 * kThreads) void k_pgemm_down_both(BDownArgs a, i
             __builtin_amdgcn_sched_barrier(0);
             if (i + 3 < n) load(i + 3, u ^ 1);
           }
-          // the next half of the table, a barrier before its first use
-          const int c = i + 3 - nh;
-          if (c >= 0 && c % kDcTab == kDcTab - 2 && c + 2 < nc) fill(c + 2);
+          if (LONG) {   // the next half of the table, a barrier before its first use
+            const int c = i + 3 - nh;
+            if (c >= 0 && c % kDcTab == kDcTab - 2 && c + 2 < nc) fill(c + 2);
+          }
           lds_barrier();
         }
       }
@@ -2170,10 +2173,15 @@ int batch_ffn(const uint16_t* x, int M, const uint16_t* norm_w, float eps, const
     // one launch for both downs (128- or 64-token tiles): one partial sum per range
     const int splits = p.both_splits;
     const dim3 grid(16 * p.pmt * splits);
+    // the table holds a range of any list this long; refilling it where it
+    // need not be cost 0.5-0.7 % of a layer (64 and 512 tokens)
+    const bool whole = (cap + kDcItems - 1) / kDcItems <= 2 * kDcTab * splits;
     if (p.pms == 4)
-      hipLaunchKernelGGL((k_pgemm_down_both<4>), grid, dim3(2 * kThreads), 0, st, da, p.pmt, splits);
+      hipLaunchKernelGGL((whole ? k_pgemm_down_both<4, false> : k_pgemm_down_both<4, true>), grid,
+                         dim3(2 * kThreads), 0, st, da, p.pmt, splits);
     else
-      hipLaunchKernelGGL((k_pgemm_down_both<2>), grid, dim3(2 * kThreads), 0, st, da, p.pmt, splits);
+      hipLaunchKernelGGL((whole ? k_pgemm_down_both<2, false> : k_pgemm_down_both<2, true>), grid,
+                         dim3(2 * kThreads), 0, st, da, p.pmt, splits);
     OI2_CHECK_LAUNCH();
     final_add(splits);
     OI2_CHECK_LAUNCH();

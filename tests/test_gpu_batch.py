@@ -375,30 +375,31 @@ def test_batch_is_bit_reproducible(dev, layer25, B):
             assert_ffn_close(runs[0][1].cpu().numpy(), ref, what=f"B={B} cold only against the oracle")
 
 
-@pytest.mark.parametrize("M,n_chunks", [(1160, 1), (1160, 56), (130 * 8, 1)])
-def test_joint_down_over_long_ranges(dev, M, n_chunks):
+@pytest.mark.parametrize("M,n_chunks,n", [(1160, 1, 5500), (1160, 56, 5500), (130 * 8, 1, 5500), (1160, 1, 4096),
+                                         (1160, 1, 4097)])
+def test_joint_down_over_long_ranges(dev, M, n_chunks, n):
     """Token counts whose down runs over one or two ranges of the whole active
-    list, so that a range passes the 2048 and 4096 items of its record offset
-    table: 5500 records in no order, some of them absent, as one dense list or
-    in 56 chunks.  Every 37th token against float32 torch over the same
+    list, so that a range passes half and the whole of its 4096-item record
+    offset table, or just fits it: n records in no order, some of them absent,
+    as one dense list or in 56 chunks.  Every 37th token against float32 torch over the same
     dequantised weights."""
     g = torch.Generator(device=dev).manual_seed(91)
     lay = SyntheticLayer(g, 6144, 200, device=dev)
     n_rec = lay.records.shape[0]
-    slots = torch.randperm(n_rec, generator=g, device=dev)[:5500].int()
+    slots = torch.randperm(n_rec, generator=g, device=dev)[:n].int()
     slots[::501] = -1
     valid = slots[slots >= 0]
     sec = _section(lay)
     if n_chunks == 1:
         cold = ColdNeurons.from_slots(sec, slots)
     else:
-        counts = torch.full((n_chunks,), 5500 // n_chunks, dtype=torch.int32, device=dev)
-        counts[3] += 5500 - int(counts.sum())
+        counts = torch.full((n_chunks,), n // n_chunks, dtype=torch.int32, device=dev)
+        counts[3] += n - int(counts.sum())
         pad = torch.full((n_chunks, 256), 7, dtype=torch.int32, device=dev)
         at = 0
-        for c, n in enumerate(counts.tolist()):
-            pad[c, :n] = slots[at:at + n]
-            at += n
+        for c, k in enumerate(counts.tolist()):
+            pad[c, :k] = slots[at:at + k]
+            at += k
         cold = ColdNeurons(sec, pad.reshape(-1), counts, n_chunks, 256)
     x = torch.randn((M, H), generator=g, device=dev).half()
     _, y32 = _ffn(x, lay.norm_w, EPS, lay.hot, cold, "silu", False, False, want_y32=True)
