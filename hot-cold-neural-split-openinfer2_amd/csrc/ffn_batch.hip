@@ -1097,8 +1097,8 @@ __global__ __launch_bounds__(kThreads) void k_pgemm_down_cold(BDownArgs a, int m
 // loaded two ahead and go through two LDS buffers, one barrier per block;
 // a buffer holds either kind.  (With 4 waves doing both, 512 tokens took
 // 4219 against 3958 us per 32 layers, 64 tokens 1868 against 1834.)
-// LONG: the range may have more blocks than the record offset table, whose
-// halves are then refilled in turn as the loop goes.
+// LONG: the range may have more blocks than the record offset table; the table
+// then has a second half, and the two are refilled in turn as the loop goes.
 template <int MS, bool LONG>
 __global__ __launch_bounds__(2 * kThreads) void k_pgemm_down_both(BDownArgs a, int mt, int splits) {
   constexpr int NB = 2;
@@ -1106,7 +1106,7 @@ __global__ __launch_bounds__(2 * kThreads) void k_pgemm_down_both(BDownArgs a, i
   constexpr int kColdT = 256 * kLdC * 2, kColdH = 32 * MS * kLdC * 2;
   constexpr int kBuf = kHotA + kHotB > kColdT + kColdH ? kHotA + kHotB : kColdT + kColdH;
   __shared__ __attribute__((aligned(16))) uint8_t smem[2 * kBuf];
-  __shared__ uint32_t s_rec[2 * kDcTab * kDcItems];   // record offsets of the range's blocks
+  __shared__ uint32_t s_rec[(LONG ? 2 : 1) * kDcTab * kDcItems];   // record offsets of the range's blocks
   __shared__ __attribute__((aligned(16))) uint16_t s_sc[4 * kDcItems];
   const int b = blockIdx.x;
   const int q = b >> 3, per = mt * splits;
@@ -2175,7 +2175,7 @@ int batch_ffn(const uint16_t* x, int M, const uint16_t* norm_w, float eps, const
     const dim3 grid(16 * p.pmt * splits);
     // the table holds a range of any list this long; refilling it where it
     // need not be cost 0.5-0.7 % of a layer (64 and 512 tokens)
-    const bool whole = (cap + kDcItems - 1) / kDcItems <= 2 * kDcTab * splits;
+    const bool whole = (cap + kDcItems - 1) / kDcItems <= kDcTab * splits;
     if (p.pms == 4)
       hipLaunchKernelGGL((whole ? k_pgemm_down_both<4, false> : k_pgemm_down_both<4, true>), grid,
                          dim3(2 * kThreads), 0, st, da, p.pmt, splits);

@@ -375,12 +375,12 @@ def test_batch_is_bit_reproducible(dev, layer25, B):
             assert_ffn_close(runs[0][1].cpu().numpy(), ref, what=f"B={B} cold only against the oracle")
 
 
-@pytest.mark.parametrize("M,n_chunks,n", [(1160, 1, 5500), (1160, 56, 5500), (130 * 8, 1, 5500), (1160, 1, 4096),
-                                         (1160, 1, 4097)])
+@pytest.mark.parametrize("M,n_chunks,n", [(1160, 1, 5500), (1160, 56, 5500), (130 * 8, 1, 5500), (1160, 1, 2048),
+                                         (1160, 1, 2049), (1160, 1, 4097)])
 def test_joint_down_over_long_ranges(dev, M, n_chunks, n):
     """Token counts whose down runs over one or two ranges of the whole active
-    list, so that a range passes half and the whole of its 4096-item record
-    offset table, or just fits it: n records in no order, some of them absent,
+    list, so that a range passes one and two halves of 2048 items of its record
+    offset table, or just fits one: n records in no order, some of them absent,
     as one dense list or in 56 chunks.  Every 37th token against float32 torch over the same
     dequantised weights."""
     g = torch.Generator(device=dev).manual_seed(91)
