@@ -1,10 +1,11 @@
 // Grouped-query attention for prompts on gfx950's matrix cores: the
 // projections and the attention of GroupedQueryAttention.forward
-// (engine.py:90-125) for calls with many token rows.
+// (engine.py:90-125) for calls with several token rows.
 //
 //   k_proj       C = X W^T, fp16 rows times fp8 e4m3fn weights (widened
 //                exactly to fp16), fp32 sums; epilogue q / k / v (RoPE, q to a
 //                buffer, k and v into the cache) or o_proj (out and x + out)
+//   k_proj_few   the same for 6 to 32 rows
 //   k_flash      attention of 64 query rows of a head per workgroup over the
 //                cache positions they see
 //
@@ -715,9 +716,10 @@ __global__ __launch_bounds__(128 * NK, 4 / NK) void k_flash(FlashArgs a, int n_q
 }  // namespace
 
 // Up to 32 rows (16 with 96 heads, whose 768 workgroups of two token tiles take
-// longer: a layer at 32 rows 105 against 92 us) k_proj_few.  From there the smallest tile whose tiles fit one workgroup per CU (64 rows, else
-// 128 rows, on 128-wide K blocks: three deep buffers of one workgroup fill a
-// CU's LDS); past that 128 rows on 64-wide K blocks, two workgroups a CU.
+// longer: a layer at 32 rows 105 against 92 us) k_proj_few.  From there the
+// smallest tile whose tiles fit one workgroup per CU (64 rows, else 128 rows,
+// on 128-wide K blocks: three deep buffers of one workgroup fill a CU's LDS);
+// past that 128 rows on 64-wide K blocks, two workgroups a CU.
 // Measured, q / k / v (48 heads) and o_proj (32 heads) in us:
 //   rows   64-row        128-row       128-row, 64-wide K
 //   100    18.3  15.8    26.9  23.6    28.1  25.2

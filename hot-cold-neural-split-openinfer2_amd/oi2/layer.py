@@ -221,7 +221,7 @@ def sparse_ffn(x: torch.Tensor, activation: str, act_on_both: bool,
       * the reference's own tensors (what SparseFFNLayer and read_neurons
         hand it): gate/up (n, H), down (H, n), fp16 (the widened hot file),
         fp32 (dequantised cold records) or bf16 - computed by the dense-weight
-        HIP GEMV kernels (oi2_sparse_ffn_dense);
+        HIP kernels (oi2_sparse_ffn_dense);
       * this library's compact handles: the whole hot half as one HotWeights
         in ``gate_hot`` (fp8 in HBM) and the whole cold half as one
         ColdNeurons in ``gate_cold`` (INT4 records + active list), with the
