@@ -20,10 +20,10 @@
 //   k_attn_gemv (out)  out = fp16(attn W_o^T) (engine.py:122-123), and
 //                      optionally x + out in the same pass
 //
-// Rounding follows the reference's fp16 tensors: x_n, q, k, v, the RoPE
-// products, sums and differences, the attention output and out are each
-// rounded to fp16 where the reference's fp16 ops round them; dot products
-// accumulate in fp32.
+// Rounding follows the reference's fp16 tensors: x_n, q, k, v, the RoPE sums
+// and their sine products (rope_f16; the cosine products stay exact in their
+// fma), the attention output and out are each rounded to fp16; dot products
+// accumulate in fp32, in an order that depends on the kernel.
 //
 // Cache layout: k_cache, v_cache (batch, n_kv, cap, 128) fp16, the
 // reference's (B, n_kv, S, D) tensors with room for cap positions.
@@ -278,11 +278,9 @@ __global__ __launch_bounds__(kThreads) void k_attn_gemv(GemvArgs a) {
   const int b = row / a.seq, t = row - b * a.seq;
   float o0 = y0, o1 = y1;
   if (hb < a.blocks0 + a.blocks1) {
-    // engine.py:150-157: cat(x1 cos - x2 sin, x1 sin + x2 cos), the tables
-    // cast to fp16 and every product and sum an fp16 op
-    const float c = round_f16(a.cos[t * kHalf + j]), s = round_f16(a.sin[t * kHalf + j]);
-    o0 = round_f16(round_f16(y0 * c) - round_f16(y1 * s));
-    o1 = round_f16(round_f16(y0 * s) + round_f16(y1 * c));
+    const RopePair o = rope_f16((_Float16)y0, (_Float16)y1, (_Float16)a.cos[t * kHalf + j], (_Float16)a.sin[t * kHalf + j]);
+    o0 = (float)o.a;
+    o1 = (float)o.b;
   }
   uint16_t* dst;
   if (hb < a.blocks0) {

@@ -8,6 +8,19 @@ namespace oi2 {
 
 constexpr int kHeadDim = 128;                 // head_dim (engine.py:72: hidden / n_q)
 
+// RoPE of the pair (x1, x2) at angle table entries (c, s), all fp16
+// (engine.py:150-157: cat(x1 cos - x2 sin, x1 sin + x2 cos) as fp16 ops).  Each
+// sum takes its sine product rounded to fp16 and its cosine product exact, and
+// is rounded once.  Every projection kernel uses this one form, so that a token
+// gets the same q and k whichever of them a call's row count picks; written
+// out with fma, because left to contraction the kernels could differ.
+struct RopePair {
+  _Float16 a, b;
+};
+__device__ __forceinline__ RopePair rope_f16(_Float16 x1, _Float16 x2, _Float16 c, _Float16 s) {
+  return {__builtin_elementwise_fma(x1, c, -(x2 * s)), __builtin_elementwise_fma(x2, c, x1 * s)};
+}
+
 // Rows of x times weight blocks of 128 rows (one head each): q / k / v with
 // RoPE, q to a buffer and k, v into the cache (mode 0), or o_proj (mode 1).
 struct ProjArgs {

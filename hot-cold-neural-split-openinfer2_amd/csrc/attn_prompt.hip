@@ -9,8 +9,8 @@
 //   k_flash      attention of 64 query rows of a head per workgroup over the
 //                cache positions they see
 //
-// Rounded to fp16: x_n, q, k, v before and after RoPE, the attention output
-// and out; everything between them is fp32.
+// Rounded to fp16: x_n, q, k, v before and after RoPE (rope_f16), the attention
+// output and out; everything between them is fp32.
 #include "attn_kernels.h"
 #include "capi_util.h"
 #include "decode_util.h"
@@ -283,23 +283,22 @@ __global__ __launch_bounds__(256, KB == 64 ? 2 : 1) void k_proj(ProjArgs a, int 
     }
     const int bt = row / a.seq, t = row - bt * a.seq;
     if (rot) {
-      // engine.py:150-157: cat(x1 cos - x2 sin, x1 sin + x2 cos), the tables
-      // cast to fp16; products and sum in fp32, rounded once to fp16
       const f32x4_a4* pc = reinterpret_cast<const f32x4_a4*>(a.cos + (size_t)t * kHalfHead + j);
       const f32x4_a4* ps = reinterpret_cast<const f32x4_a4*>(a.sin + (size_t)t * kHalfHead + j);
       const f32x4 c[2] = {pc[0], pc[1]}, s[2] = {ps[0], ps[1]};
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
-        float o0[2], o1[2];
+        const f16x2 x0 = as_f16x2(v0[d]), x1 = as_f16x2(v1[d]);
+        f16x2 o0, o1;
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
-          const float x0 = k ? half_hi(v0[d]) : half_lo(v0[d]), x1 = k ? half_hi(v1[d]) : half_lo(v1[d]);
-          const float cc = round_f16(c[d >> 1][2 * (d & 1) + k]), ss = round_f16(s[d >> 1][2 * (d & 1) + k]);
-          o0[k] = x0 * cc - x1 * ss;
-          o1[k] = x0 * ss + x1 * cc;
+          const int e = 2 * (d & 1) + k;
+          const RopePair o = rope_f16(x0[k], x1[k], (_Float16)c[d >> 1][e], (_Float16)s[d >> 1][e]);
+          o0[k] = o.a;
+          o1[k] = o.b;
         }
-        v0[d] = pack_f16x2(o0[0], o0[1]);
-        v1[d] = pack_f16x2(o1[0], o1[1]);
+        v0[d] = __builtin_bit_cast(uint32_t, o0);
+        v1[d] = __builtin_bit_cast(uint32_t, o1);
       }
     }
     uint16_t* dst;
@@ -406,9 +405,10 @@ __global__ __launch_bounds__(kFewThreads, 4) void k_proj_few(ProjArgs a) {
     const int bt = row / a.seq, tt = row - bt * a.seq;
     float o0 = y0, o1 = y1;
     if (hb < a.blocks0 + a.blocks1) {
-      const float c = round_f16(a.cos[(size_t)tt * kHalfHead + j]), s = round_f16(a.sin[(size_t)tt * kHalfHead + j]);
-      o0 = y0 * c - y1 * s;
-      o1 = y0 * s + y1 * c;
+      const size_t e = (size_t)tt * kHalfHead + j;
+      const RopePair o = rope_f16((_Float16)y0, (_Float16)y1, (_Float16)a.cos[e], (_Float16)a.sin[e]);
+      o0 = (float)o.a;
+      o1 = (float)o.b;
     }
     uint16_t* dst;
     if (hb < a.blocks0) {
