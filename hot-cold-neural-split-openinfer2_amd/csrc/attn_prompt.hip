@@ -469,7 +469,8 @@ __global__ __launch_bounds__(128 * NK, 4 / NK) void k_flash(FlashArgs a, int n_q
   __shared__ __align__(1024) uint8_t sK0[kFP * 256], sK1[kFP * 256];
   __shared__ __align__(1024) uint8_t sV0[kHeadDim * kFP * 2], sV1[kHeadDim * kFP * 2];
   __shared__ float s_m[kW][32], s_l[kW][32];
-  __shared__ uint32_t s_bad[2][NK];            // per buffer: positions of the tile with a non-finite v
+  __shared__ uint32_t s_bad[3][NK];            // tile kt % 3: its positions with a non-finite v
+  __shared__ uint32_t s_redo;
   const int b = blockIdx.x;
   // the four heads of blocks 8 apart share an XCD: with up to 8 kv heads they
   // are of one kv head, whose K and V its L2 then holds
@@ -507,11 +508,16 @@ __global__ __launch_bounds__(128 * NK, 4 / NK) void k_flash(FlashArgs a, int n_q
   };
   // whether some row of the workgroup must not see some position of tile kt
   auto masked = [&](int kt) { return a.causal && (kt + 1) * kFP > a.past + q0 + 1; };
-  auto store_v = [&](int kt, int buf, uint8_t* sV) {
-    if (masked(kt)) {
-      // a masked position's probability is 0, and 0 times a non-finite v would
-      // spoil rows that do not see it: such v go in as 0 here, and their
-      // positions are noted and added one by one to the rows that see them
+  // A non-finite v cannot go through the products: a masked position's
+  // probability is 0, and so is the low part of one that fp16 holds exactly, and
+  // 0 times it would be NaN where the row does not see it, or sees infinity.  It
+  // always leaves a non-finite sum, so the tiles are run without looking for it;
+  // a workgroup that ends with such a sum runs them once more with `careful`.
+  bool careful = false;
+  auto store_v = [&](int kt, uint8_t* sV) {
+    if (careful) {
+      // non-finite v go in as 0, and their positions are noted and added one by
+      // one to the rows that see them
       uint32_t bad = 0;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
@@ -522,7 +528,7 @@ __global__ __launch_bounds__(128 * NK, 4 / NK) void k_flash(FlashArgs a, int n_q
           vr[i][d] = x & ~(lo | hi);
           if (lo | hi) bad |= 1u << i;
         }
-      if (bad) atomicOr(&s_bad[buf][pg >> 3], bad << (4 * (pg & 7)));
+      if (bad) atomicOr(&s_bad[kt % 3][pg >> 3], bad << (4 * (pg & 7)));
     }
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
@@ -549,19 +555,14 @@ __global__ __launch_bounds__(128 * NK, 4 / NK) void k_flash(FlashArgs a, int n_q
   const float ninf = -__builtin_inff();
 
   f32x16 o[4];
-#pragma unroll
-  for (int d = 0; d < 4; ++d) o[d] = f32x16{};
-  float m = ninf, lsum = 0.0f;                            // of this lane's positions; m of both halves
+  float m, lsum;                                          // of this lane's positions; m of both halves
 
-  if (t < 2 * NK) s_bad[t / NK][t % NK] = 0;
-  load_k(0, sK0);
-  load_v(0);
-  __syncthreads();                                        // s_bad is cleared
-  store_v(0, 0, sV0);
-
-  auto tile = [&](int kt, int buf, const uint8_t* cK, const uint8_t* cV, uint8_t* nK, uint8_t* nV) {
+  auto tile = [&](int kt, const uint8_t* cK, const uint8_t* cV, uint8_t* nK, uint8_t* nV) {
     // K's DMAs (the only loads in flight) and V's stores of this tile are done
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // of the tile before, which every wave is done with; the one after the
+    // next's, a barrier before its first use
+    if (careful && t < NK) s_bad[(kt + 2) % 3][t] = 0;
     const bool more = kt + 1 < n_kt;
     if (more) {
       load_k(kt + 1, nK);
@@ -633,9 +634,9 @@ __global__ __launch_bounds__(128 * NK, 4 / NK) void k_flash(FlashArgs a, int n_q
           o[d] = mfma32(vf, ph[s2], o[d]);
           o[d] = mfma32(vf, pl[s2], o[d]);
         }
-      if (masked(kt)) {
-        uint32_t bad = s_bad[buf][kv];
-        while (bad) {                                     // workgroup-uniform, hardly ever entered
+      if (careful) {
+        uint32_t bad = s_bad[kt % 3][kv];
+        while (bad) {
           const int pos = __builtin_ctz(bad);             // of this wave's 32
           bad &= bad - 1;
           const int jj = 4 * (pos >> 3) + (pos & 3), hh = (pos >> 2) & 1;
@@ -655,15 +656,40 @@ __global__ __launch_bounds__(128 * NK, 4 / NK) void k_flash(FlashArgs a, int n_q
       }
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (more) store_v(kt + 1, buf ^ 1, nV);
+    if (more) store_v(kt + 1, nV);
   };
+  if (t == 0) s_redo = 0u;                                // set after the first tile's barrier at the earliest
 #pragma unroll 1
-  for (int kt = 0; kt < n_kt; kt += 2) {
-    tile(kt, 0, sK0, sV0, sK1, sV1);
-    if (kt + 1 < n_kt) tile(kt + 1, 1, sK1, sV1, sK0, sV0);
+  for (;;) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) o[d] = f32x16{};
+    m = ninf;
+    lsum = 0.0f;
+    load_k(0, sK0);
+    load_v(0);
+    if (careful) {
+      if (t < 2 * NK) s_bad[t / NK][t % NK] = 0;
+      __syncthreads();
+    }
+    store_v(0, sV0);
+#pragma unroll 1
+    for (int kt = 0; kt < n_kt; kt += 2) {
+      tile(kt, sK0, sV0, sK1, sV1);
+      if (kt + 1 < n_kt) tile(kt + 1, sK1, sV1, sK0, sV0);
+    }
+    if (!careful) {
+      float z = 0.0f;                                     // NaN once a sum is not finite
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) z = fmaf(o[d][j], 0.0f, z);
+      if (__any(z != z) && l == 0) s_redo = 1u;
+    }
+    __syncthreads();                                      // the tiles are no longer read
+    if (careful || s_redo == 0u) break;
+    careful = true;
   }
   lsum += __shfl_xor(lsum, 32);                           // of the wave's positions
-  __syncthreads();                                        // the tiles are no longer read
   // wave (qs, kv) finishes dims kOut kv .. of its rows: every wave leaves its
   // sums of each wave's dims in that wave's buffer (a wave with no position
   // has m = -inf)

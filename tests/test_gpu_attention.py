@@ -293,6 +293,52 @@ def test_a_prompt_row_does_not_see_later_non_finite_values(dev, bad):
     assert not torch.isfinite(out[0, bad:]).any()
 
 
+def _infinite_setup(dev, n_kv):
+    """Weights with which a token of ones has v = 4096 * 24, infinite in fp16,
+    in every dim, and every output is the sum of the attention's dims: rows
+    that see the token come out as inf, not NaN."""
+    w = _weights(dev, n_kv, seed=91)
+    w["layer_000.v_proj"] = torch.full((n_kv * D, H), 24.0, device=dev).to(torch.float8_e4m3fn)
+    w["layer_000.o_proj"] = torch.full((H, H), 2.0 ** -9, device=dev).to(torch.float8_e4m3fn)
+    w["layer_000.input_layernorm"] = torch.ones(H, dtype=torch.float16, device=dev)
+    return w
+
+
+@pytest.mark.parametrize("T,bad", [(100, 40), (200, 5), (200, 130), (600, 5), (600, 300), (600, 599)])
+def test_prompt_rows_that_see_an_infinite_value_are_infinite(dev, T, bad):
+    """Tiles of positions that some row of a workgroup does not see, and tiles that every row
+    of a workgroup sees (where an infinite v times the zero low part of its
+    probability must not become NaN), with four position parts a workgroup
+    (up to 512 rows) and with two."""
+    n_kv = 8
+    w = _infinite_setup(dev, n_kv)
+    cos, sin = oi2.rope_tables(T, D, 1e6, device=dev)
+    x = torch.randn((1, T, H), generator=torch.Generator(device=dev).manual_seed(92), device=dev).half()
+    x[0, bad] = 1.0
+    out, (_, v) = oi2.GroupedQueryAttention(0, w, _cfg(n_kv))(x, cos, sin)
+    cut, _ = oi2.GroupedQueryAttention(0, w, _cfg(n_kv))(x[:, :bad].contiguous(), cos, sin)
+    assert torch.isposinf(v[0, :, bad]).all() and torch.isfinite(v[0, :, :bad]).all()
+    assert torch.isposinf(out[0, bad:]).all()
+    assert_ffn_close(out[0, :bad].float().cpu().numpy(), cut[0].float().cpu().numpy(), tol=2e-3, what="rows before")
+
+
+@pytest.mark.parametrize("T,past,at,value", [(16, 300, 7, "inf"), (70, 300, 290, "-inf"), (600, 200, 130, "inf"),
+                                             (16, 300, 100, "nan")])
+def test_rows_over_a_cache_with_a_non_finite_value(dev, T, past, at, value):
+    """A chunk over a cache (every row sees every position) one of whose v is
+    not finite: every output is that value."""
+    n_kv = 8
+    w = _infinite_setup(dev, n_kv)
+    cos, sin = oi2.rope_tables(past + T, D, 1e6, device=dev)
+    x = torch.randn((1, T, H), generator=torch.Generator(device=dev).manual_seed(93), device=dev).half()
+    k, v = _rand_cache(dev, 1, n_kv, past, seed=94)
+    v[0, :, at] = float(value)
+    out, _ = oi2.GroupedQueryAttention(0, w, _cfg(n_kv))(x, cos[past:], sin[past:], (k, v))
+    want = torch.full_like(out, float(value))
+    assert torch.equal(torch.nan_to_num(out, nan=1.0, posinf=2.0, neginf=3.0),
+                       torch.nan_to_num(want, nan=1.0, posinf=2.0, neginf=3.0))
+
+
 @pytest.mark.parametrize("rows", [6, 17, 33, 400, 700])
 def test_a_token_gets_the_same_k_and_v_whichever_projection_runs(dev, rows):
     """The cached k and v of five tokens from a call of their own and from one
