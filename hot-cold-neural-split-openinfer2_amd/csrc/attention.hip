@@ -349,20 +349,20 @@ __global__ __launch_bounds__(kThreads) void k_attn_sdpa(SdpaArgs a) {
   struct Rows {
     u32x4 k[STEPS], v[STEPS];
   };
-  // chunk c: positions base + 4 kPW c + 4 it + k, those past n_r clamped
+  // chunk c: positions base + 4 kPW c + 4 it + k; those past n_r read zero
+  // through the descriptors' range (clamped to the last position, its v, where
+  // it is infinite, times their probability 0 would be NaN) and score -inf
+  const rsrc_t rk = make_rsrc(a.k_cache + head * kHd, (uint32_t)n_r * kHd * 2);
+  const rsrc_t rv = make_rsrc(a.v_cache + head * kHd, (uint32_t)n_r * kHd * 2);
   auto load = [&](int c, Rows& x) {
     const int p0 = base + 4 * kPW * c + k;
 #pragma unroll
     for (int it = 0; it < STEPS; ++it) {
-      const int p = p0 + 4 * it;
-      const int pc = p < n_r ? p : n_r - 1;
-      x.k[it] = *reinterpret_cast<const u32x4*>(a.k_cache + (head + pc) * kHd + 8 * jj);
+      x.k[it] = __builtin_amdgcn_raw_buffer_load_b128(rk, (uint32_t)(p0 + 4 * it) * (kHd * 2) + 16 * jj, 0, 0);
     }
 #pragma unroll
     for (int it = 0; it < STEPS; ++it) {
-      const int p = p0 + 4 * it;
-      const int pc = p < n_r ? p : n_r - 1;
-      x.v[it] = *reinterpret_cast<const u32x4*>(a.v_cache + (head + pc) * kHd + 8 * jj);
+      x.v[it] = __builtin_amdgcn_raw_buffer_load_b128(rv, (uint32_t)(p0 + 4 * it) * (kHd * 2) + 16 * jj, 0, 0);
     }
   };
 

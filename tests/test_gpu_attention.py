@@ -339,6 +339,19 @@ def test_rows_over_a_cache_with_a_non_finite_value(dev, T, past, at, value):
                        torch.nan_to_num(want, nan=1.0, posinf=2.0, neginf=3.0))
 
 
+@pytest.mark.parametrize("past", [300, 1500, 1535, 6399, 6400, 6655])
+def test_a_decoded_token_with_an_infinite_value(dev, past):
+    """One token whose own v is infinite, at every place of the last split
+    (short spans, one-shot and looping splits): the output is infinite.  The
+    loads past the span must not meet that v with a probability of 0."""
+    n_kv = 8
+    w = _infinite_setup(dev, n_kv)
+    cos, sin = oi2.rope_tables(past + 1, D, 1e6, device=dev)
+    x = torch.ones((1, 1, H), device=dev).half()
+    out, _ = oi2.GroupedQueryAttention(0, w, _cfg(n_kv))(x, cos[past:], sin[past:], _rand_cache(dev, 1, n_kv, past, seed=95))
+    assert torch.isposinf(out).all()
+
+
 @pytest.mark.parametrize("rows", [6, 17, 33, 400, 700])
 def test_a_token_gets_the_same_k_and_v_whichever_projection_runs(dev, rows):
     """The cached k and v of five tokens from a call of their own and from one
