@@ -1918,7 +1918,33 @@ static int cold_down_splits(int M, int cap) {
   return std::max(min_splits, std::min(n_blk, std::max(1, 256 / (16 * mtc))));
 }
 
-static BatchPlan batch_plan(int M, int n_hot, int cap) {
+// K ranges of the joint down, each one partial sum of y.  While its tiles
+// leave room in a round of one workgroup per CU: as many as fit the round (but
+// no more than the larger half has blocks).  From 1025 tokens one range fills
+// at least half a round, and more of them only pay where they trim the last
+// round: the whole K takes 1.14 us a round per hot block and 1.28 us per cold
+// block, a range's partial sum 6.9 ns per token to store and add (fitted to
+// 1100 to 4100 tokens, 1 to 8 ranges).  The blocks are the capacity's where the
+// list is dense, and so as long as it was made; a chunked list has room for
+// every neuron and hardly ever more than a sixteenth of them active.  Layers
+// with 3584 hot neurons, 1 range and the taken number: 1100 tokens, 4301 in the
+// list, 321 and 297 us (3 ranges); 540 of 14336, 180 and 178 (3); 1300 tokens,
+// 540 of 14336, 184 (1; with the 7 ranges that one per 2048 of the capacity
+// makes, 226); 2100 tokens, 4301, 599 and 538 (3); 540, 305 and 297 (2).
+static int joint_down_splits(int M, int pmt, int hot_blocks, int cap, bool dense) {
+  const int n_blk = (cap + kDcItems - 1) / kDcItems, tiles = 16 * pmt, want = std::max(1, 256 / tiles);
+  const int fit = std::max(std::min(hot_blocks, want), std::min(n_blk, want));
+  if (want > 1) return fit;
+  const double round_us = 1.14 * hot_blocks + 1.28 * (dense ? n_blk : (n_blk + 15) / 16);
+  auto cost = [&](int n) { return (double)((tiles * n + 255) / 256) / n * round_us + 6.9e-3 * M * n; };
+  int best = fit;
+  for (int n = fit + 1; n <= 4; ++n)
+    if (cost(n) < cost(best)) best = n;
+  return best;
+}
+
+// `dense`: the active list is one chunk, its capacity its length.
+static BatchPlan batch_plan(int M, int n_hot, int cap, bool dense) {
   BatchPlan p{};
   p.M = M;
   p.Mpad = (M + kBM - 1) / kBM * kBM;
@@ -1955,20 +1981,16 @@ static BatchPlan batch_plan(int M, int n_hot, int cap) {
   o = align256(o + 16);
   p.off_y = o;
   // up to 16 tokens: y (M, H); from 17: one (M, H) partial sum per down range
-  // (separate hot and cold downs, or the ranges of the joint one)
+  // (the joint down's, for either kind of list, or those of the only half)
   p.both_splits = 0;
+  int y_parts = 1;
   if (M > kSkinnyMax && n_hot > 0 && cap > 0) {
-    // about 256 workgroups, whatever the list's capacity: a drop-in layer's
-    // list has room for every neuron, and one range per 2048 of it made a
-    // 1300-token prompt with 540 active records write and add seven partial
-    // sums (down 84 us, final add 26; one range: 70 and 9)
-    const int n_blk = (cap + kDcItems - 1) / kDcItems, want = std::max(1, 256 / (16 * p.pmt));
-    p.both_splits = std::max(std::min(p.hot_blocks, want), std::min(n_blk, want));
+    p.both_splits = joint_down_splits(M, p.pmt, p.hot_blocks, cap, dense);
+    y_parts = std::max(p.both_splits, joint_down_splits(M, p.pmt, p.hot_blocks, cap, !dense));
+  } else if (M > kSkinnyMax) {
+    y_parts = n_hot > 0 ? p.hot_splits : cap > 0 ? cold_down_splits(M, cap) : 1;
   }
-  const int y_parts = M <= kSkinnyMax ? 1
-                                      : std::max(p.both_splits, (n_hot > 0 ? p.hot_splits : 0) +
-                                                                    (cap > 0 ? cold_down_splits(M, cap) : 0));
-  o = align256(o + (size_t)std::max(1, y_parts) * M * kH * 4);
+  o = align256(o + (size_t)y_parts * M * kH * 4);
   p.cold_splits = (M <= kSkinnyMax && cap > 0) ? cold_down_splits(M, cap) : 0;
   p.off_part = o;
   o = align256(o + (size_t)p.cold_splits * kH * 16 * 4);
@@ -2003,7 +2025,7 @@ static MupTiles mup_tiles(const BatchPlan& p) {
   return m;
 }
 
-size_t batch_ws_bytes(int M, int n_hot, int cap) { return batch_plan(M, n_hot, cap).bytes; }
+size_t batch_ws_bytes(int M, int n_hot, int cap) { return batch_plan(M, n_hot, cap, true).bytes; }
 
 static void launch_skinny(const BUpArgs& ua, const BDownArgs& da, bool up, const uint16_t* x,
                           const uint16_t* norm_w, float eps, hipStream_t st) {
@@ -2022,7 +2044,7 @@ int batch_ffn(const uint16_t* x, int M, const uint16_t* norm_w, float eps, const
   const int n_hot = hot ? hot->n_hot : 0;
   const bool has_cold = cold && active && cold->n_records > 0 && active->n_chunks > 0;
   const int cap = has_cold ? active->n_chunks * active->chunk : 0;
-  const BatchPlan p = batch_plan(M, n_hot, cap);
+  const BatchPlan p = batch_plan(M, n_hot, cap, has_cold && active->n_chunks == 1);
   OI2_CHECK_ARG(workspace && workspace_bytes >= p.bytes,
                 "workspace of %zu bytes is smaller than the %zu required", workspace_bytes, p.bytes);
   OI2_CHECK_ARG((uintptr_t)workspace % 256 == 0, "workspace must be 256-byte aligned");

@@ -378,9 +378,9 @@ def test_batch_is_bit_reproducible(dev, layer25, B):
 @pytest.mark.parametrize("M,n_chunks,n", [(1160, 1, 5500), (1160, 56, 5500), (130 * 8, 1, 5500), (1160, 1, 2048),
                                          (1160, 1, 2049), (1160, 1, 4097)])
 def test_joint_down_over_long_ranges(dev, M, n_chunks, n):
-    """Token counts whose down runs over one or two ranges of the whole active
-    list, so that a range passes one and two halves of 2048 items of its record
-    offset table, or just fits one: n records in no order, some of them absent,
+    """Token counts whose down runs over one range of the whole active list, so
+    that it passes one and two halves of 2048 items of its record offset table,
+    or just fits one: n records in no order, some of them absent,
     as one dense list or in 56 chunks.  Every 37th token against float32 torch over the same
     dequantised weights."""
     g = torch.Generator(device=dev).manual_seed(91)
@@ -410,3 +410,41 @@ def test_joint_down_over_long_ranges(dev, M, n_chunks, n):
     for G, U, D in (hot_dense(lay.hot), cold_dense(lay.records, valid)):
         ref = ref + (torch.nn.functional.silu(xn @ f32(G).T) * (xn @ f32(U).T)) @ f32(D).T
     assert_ffn_close(y32[rows].cpu().numpy(), ref.double().cpu().numpy(), what=f"{M} tokens, {n_chunks} chunks")
+
+
+@pytest.mark.parametrize("M,n_hot,n_chunks,n,cap", [
+    (130, 200, 1, 13000, 0), (159, 200, 56, 13000, 14336), (300, 200, 56, 13000, 14336), (512, 700, 1, 13000, 0),
+    (1024, 200, 1, 5500, 0), (1024, 200, 56, 13000, 14336), (1100, 3000, 1, 4301, 0), (1100, 3000, 56, 700, 14336),
+    (2100, 3000, 1, 8191, 0), (64, 1000, 56, 3, 14336)])
+def test_joint_down_over_several_ranges(dev, M, n_hot, n_chunks, n, cap):
+    """Several ranges of the hot blocks and of the list in one launch, uneven
+    ones and ranges of more than 2048 items (whose record offsets are refilled
+    from a block that is not the list's first) among them, for both tile sizes
+    and both kinds of list; a list far shorter than its room.  Against the sum
+    of the hot half alone and the cold half alone, whose kernels have no joint
+    ranges: the same products, fp32 sums of at most n_hot + n of them in
+    another order (1e-5 of the largest: sqrt(14000) 2^-24, twice)."""
+    g = torch.Generator(device=dev).manual_seed(97)
+    lay = SyntheticLayer(g, 14336, n_hot, device=dev)
+    n_rec = lay.records.shape[0]
+    slots = torch.randperm(n_rec, generator=g, device=dev)[:n].int()
+    slots[::501] = -1
+    sec = _section(lay)
+    if n_chunks == 1:
+        cold = ColdNeurons.from_slots(sec, slots)
+    else:
+        counts = torch.full((n_chunks,), n // n_chunks, dtype=torch.int32, device=dev)
+        counts[3] += n - int(counts.sum())
+        pad = torch.full((n_chunks, cap // n_chunks), 7, dtype=torch.int32, device=dev)
+        at = 0
+        for c, k in enumerate(counts.tolist()):
+            pad[c, :k] = slots[at:at + k]
+            at += k
+        cold = ColdNeurons(sec, pad.reshape(-1), counts, n_chunks, cap // n_chunks)
+    x = torch.randn((M, H), generator=g, device=dev).half()
+    y, hot, cd = (_ffn(x, lay.norm_w, EPS, h, c, "silu", False, False, want_y32=True)[1]
+                  for h, c in ((lay.hot, cold), (lay.hot, None), (None, cold)))
+    ref = hot + cd
+    err = float((y - ref).abs().max() / ref.abs().max())
+    print(f"[batch] M={M} n_hot={n_hot} chunks={n_chunks} n={n}: max rel err {err:.1e}", flush=True)
+    assert err <= 1e-5

@@ -260,3 +260,19 @@ def test_stream_handle_refuses_a_host_device():
     for device in (torch.device("cpu"), torch.device("meta")):
         with pytest.raises(ValueError):
             _lib.stream_handle(device)
+
+
+@pytest.mark.parametrize("M,n_hot,cap,parts", [(512, 3584, 4301, 4), (1300, 3584, 14336, 4), (1100, 3584, 4301, 3),
+                                               (1100, 1024, 640, 1), (2100, 3584, 4301, 3), (3500, 3584, 4301, 1),
+                                               (300, 3584, 0, 5), (1300, 0, 4301, 3)])
+def test_batch_workspace_holds_one_partial_sum_per_down_range(M, n_hot, cap, parts):
+    """The batch FFN's workspace: normalised rows, h of both halves, the dense
+    list, and one (M, H) fp32 partial sum per range of the down that runs -
+    joint for both halves (more ranges than fill the chip once only where they
+    trim the last round of its tiles: 1100 to 2100 tokens over a long list; a
+    capacity may be a dense list's length), else the one half's."""
+    up = lambda v, n: (v + n - 1) // n * n
+    rows = up(M, 64)
+    fixed = sum(up(b, 256) for b in (2 * M * 4096, 2 * rows * up(n_hot, 128), 2 * rows * up(cap, 128), 4 * cap, 16))
+    got = oi2.load_library().oi2_ffn_workspace_bytes(M, n_hot, cap) - fixed
+    assert got == up(4 * M * 4096 * parts, 256)
