@@ -802,16 +802,28 @@ int choose_steps(int rows, int n_kv, int n_max) {
   return 2;
 }
 
+// Whether a call's attention is the prompt attention, which walks the span in
+// one workgroup per 64 rows and head.  A handful of rows over a long span has
+// too few of those, and the split kernel is faster (whole layer, n_kv 8: 9 rows
+// over 1000 positions 49 us against 52, over 4000 73 against 90; 16 rows over
+// 4000 102 against 91, 64 rows 382 against 94; n_kv 32: 9 rows over 4000 149
+// against 91).
+bool uses_flash(int rows, int seq, int n_kv, int span) {
+  return rows <= kPromptMaxRows && seq >= kFlashSeq && span <= kFlashMaxSpan &&
+         (rows >= 16 || rows * n_kv >= 256 || span <= 512);
+}
+
 struct WsLayout {
   size_t q, attn, counters, part, total;
 };
 
 // The split partial sums: none when the span (past + seq positions) fits one
-// workgroup per query head, else the splits choose_steps picks for that span
-// (the looping kernel makes at most as many).
-WsLayout ws_layout(int rows, int n_q, int n_kv, int span) {
+// workgroup per query head or the prompt attention runs, else the splits
+// choose_steps picks for that span (the looping kernel makes at most as many).
+WsLayout ws_layout(int rows, int seq, int n_q, int n_kv, int span) {
   const int G = n_q / n_kv;
-  const int per_split = span <= kOneWgMax ? 0 : 16 * choose_steps(rows, n_kv, span);
+  const int per_split =
+      span <= kOneWgMax || uses_flash(rows, seq, n_kv, span) ? 0 : 16 * choose_steps(rows, n_kv, span);
   const size_t n_split = per_split ? (size_t)(span + per_split - 1) / per_split : 0;
   WsLayout w;
   w.q = 0;
@@ -833,7 +845,7 @@ size_t oi2_attn_workspace_bytes(int32_t batch, int32_t seq, int32_t n_q, int32_t
   if (batch <= 0 || seq <= 0 || n_q <= 0 || n_kv <= 0 || n_q % n_kv || past < 0 ||
       (int64_t)past + seq > INT32_MAX)
     return 0;
-  return ws_layout(batch * seq, n_q, n_kv, past + seq).total;
+  return ws_layout(batch * seq, seq, n_q, n_kv, past + seq).total;
 }
 
 int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_attn* w, float eps,
@@ -863,7 +875,7 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
   OI2_CHECK_ARG(out, "null output");
   OI2_CHECK_ARG((size_t)batch * n_kv * cache_cap * kHd < ((size_t)1 << 40), "cache too large");
   const int rows = batch * seq;
-  const WsLayout L = ws_layout(rows, n_q, n_kv, past + seq);
+  const WsLayout L = ws_layout(rows, seq, n_q, n_kv, past + seq);
   OI2_CHECK_ARG(workspace && workspace_bytes >= L.total, "workspace of %zu bytes, %zu needed",
                 workspace_bytes, L.total);
   // spans past the merge table are refused whichever kernels would run
@@ -902,13 +914,7 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
   g.sin = sin;
   g.n_counters = rows * n_kv;
   const bool prompt = rows >= kPromptRows && rows <= kPromptMaxRows;
-  // The prompt attention walks the span in one workgroup per 64 rows and head.
-  // A handful of rows over a long span has too few of those, and the split
-  // kernel is faster (whole layer, n_kv 8: 9 rows over 1000 positions 49 us
-  // against 52, over 4000 73 against 90; 16 rows over 4000 102 against 91,
-  // 64 rows 382 against 94; n_kv 32: 9 rows over 4000 149 against 91).
-  const bool flash = prompt && seq >= kFlashSeq && past + seq <= kFlashMaxSpan &&
-                     (rows >= 16 || rows * n_kv >= 256 || past + seq <= 512);
+  const bool flash = uses_flash(rows, seq, n_kv, past + seq);
   if (prompt) {
     // x_n into the attention output's buffer, free until the attention runs
     hipLaunchKernelGGL(k_rmsnorm, dim3(rows), dim3(kThreads), 0, st, x, w->norm_w, eps, attn);

@@ -276,3 +276,13 @@ def test_batch_workspace_holds_one_partial_sum_per_down_range(M, n_hot, cap, par
     fixed = sum(up(b, 256) for b in (2 * M * 4096, 2 * rows * up(n_hot, 128), 2 * rows * up(cap, 128), 4 * cap, 16))
     got = oi2.load_library().oi2_ffn_workspace_bytes(M, n_hot, cap) - fixed
     assert got == up(4 * M * 4096 * parts, 256)
+
+
+def test_attention_workspace_of_a_long_prompt():
+    """The prompt attention takes no split partial sums: the workspace holds q,
+    the attention output and the counters, 0.5 GB at 32768 tokens."""
+    lib = oi2.load_library()
+    for B, T, past, n_kv in [(1, 32768, 0, 8), (2, 1300, 0, 4), (1, 64, 20000, 8), (1, 9, 4000, 32)]:
+        assert lib.oi2_attn_workspace_bytes(B, T, 32, n_kv, past) <= B * T * (2 * 8192 + 4 * n_kv) + 3 * 256
+    for B, T, past, n_kv in [(1, 1, 1024, 8), (1, 9, 4000, 8), (8, 1, 1999, 8)]:   # the split kernel's partial sums
+        assert lib.oi2_attn_workspace_bytes(B, T, 32, n_kv, past) > B * T * (2 * 8192 + 4 * n_kv) + 3 * 256
