@@ -37,21 +37,17 @@ namespace {
 
 constexpr int kHd = kHeadDim;
 constexpr int kHalf = kHd / 2;
-constexpr int kMaxRows = 8;              // token rows per GEMV launch (of those past kPromptMaxRows)
 // From these rows on the projections run on the matrix cores (attn_prompt.hip),
-// behind a norm launch of their own.  A whole layer at 200 cached positions,
+// behind a norm launch of their own, below it in one GEMV launch each.  A whole layer at 200 cached positions,
 // GEMV against these: 4 rows 22.2, 23.9 us; 5 rows 24.5, 24.3; 6 rows 27.2,
-// 24.9; 8 rows 31.7, 26.9; 16 rows (two GEMV passes) 57.8, 32.5.
+// 24.9; 8 rows 31.7, 26.9; 16 rows (GEMV passes of 8) 57.8, 32.5.
 constexpr int kPromptRows = 6;
 constexpr int kFlashSeq = 9;             // rows of a sequence from which attention runs on the matrix cores
 constexpr int kFlashMaxSpan = 1 << 23;   // 32-bit byte offsets into one head's cache
-constexpr int kPromptMaxRows = 0x7FFFFFFF / (kH * 2);   // 32-bit byte offsets into the rows
-constexpr int kMinPosPerWg = 32;         // 4 waves x 2 steps of 4 positions
 constexpr int kMaxTabBytes = 64 << 10;   // the merge's m / l table in LDS
 
 struct GemvArgs {
-  const uint16_t* x;          // this launch's first input row (rows, H)
-  int row0;                   // call-wide index of that row (b * seq + t)
+  const uint16_t* x;          // input rows (rows, H)
   const uint16_t* norm_w;     // RMSNorm weight, or null: the rows are used as they are
   float eps;
   const uint8_t* w0;          // weight blocks of 128 rows (.., H), fp8 e4m3fn
@@ -261,7 +257,7 @@ __global__ __launch_bounds__(kThreads) void k_attn_gemv(GemvArgs a) {
     }
   }
   if (lane >= R) return;
-  const int row = a.row0 + lane;
+  const int row = lane;
   const float y0 = round_f16(t0), y1 = round_f16(t1);
   if (a.mode == 1) {
     uint16_t* o = a.out + (size_t)row * kH + hb * kHd + j;
@@ -751,16 +747,25 @@ void launch_gemv_r(const GemvArgs& a, int blocks, hipStream_t st) {
   hipLaunchKernelGGL(k_attn_gemv<R>, dim3(blocks * 16), dim3(kThreads), 0, st, a);
 }
 
+static_assert(kPromptRows == 6, "launch_gemv's rows");
 void launch_gemv(const GemvArgs& a, int rows, int blocks, hipStream_t st) {
   switch (rows) {
     case 1: launch_gemv_r<1>(a, blocks, st); break;
     case 2: launch_gemv_r<2>(a, blocks, st); break;
     case 3: launch_gemv_r<3>(a, blocks, st); break;
     case 4: launch_gemv_r<4>(a, blocks, st); break;
-    case 5: launch_gemv_r<5>(a, blocks, st); break;
-    case 6: launch_gemv_r<6>(a, blocks, st); break;
-    case 7: launch_gemv_r<7>(a, blocks, st); break;
-    default: launch_gemv_r<8>(a, blocks, st); break;
+    default: launch_gemv_r<5>(a, blocks, st); break;
+  }
+}
+
+// One projection of every row of a call.
+void project(ProjArgs p, const uint16_t* x, int rows, int n_heads, hipStream_t st) {
+  for (int r0 = 0; r0 < rows; r0 += kProjMaxRows) {
+    p.x = x + (size_t)r0 * kH;
+    p.row0 = r0;
+    p.rows = rows - r0 < kProjMaxRows ? rows - r0 : kProjMaxRows;
+    launch_proj(p, n_heads, st);
+    p.n_counters = 0;                    // cleared by the first launch
   }
 }
 
@@ -809,7 +814,7 @@ int choose_steps(int rows, int n_kv, int n_max) {
 // 4000 102 against 91, 64 rows 382 against 94; n_kv 32: 9 rows over 4000 149
 // against 91).
 bool uses_flash(int rows, int seq, int n_kv, int span) {
-  return rows <= kPromptMaxRows && seq >= kFlashSeq && span <= kFlashMaxSpan &&
+  return rows <= kProjMaxRows && seq >= kFlashSeq && span <= kFlashMaxSpan &&
          (rows >= 16 || rows * n_kv >= 256 || span <= 512);
 }
 
@@ -893,35 +898,13 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
   uint32_t* counters = reinterpret_cast<uint32_t*>(ws + L.counters);
   float* part = reinterpret_cast<float*>(ws + L.part);
 
-  GemvArgs g{};
-  g.norm_w = w->norm_w;
-  g.eps = eps;
-  g.w0 = w->wq;
-  g.w1 = w->wk;
-  g.w2 = w->wv;
-  g.blocks0 = n_q;
-  g.blocks1 = n_kv;
-  g.mode = 0;
-  g.q = qb;
-  g.q_width = n_q * kHd;
-  g.k_cache = k_cache;
-  g.v_cache = v_cache;
-  g.n_kv = n_kv;
-  g.cap = cache_cap;
-  g.past = past;
-  g.seq = seq;
-  g.cos = cos;
-  g.sin = sin;
-  g.n_counters = rows * n_kv;
-  const bool prompt = rows >= kPromptRows && rows <= kPromptMaxRows;
+  const bool prompt = rows >= kPromptRows;
   const bool flash = uses_flash(rows, seq, n_kv, past + seq);
   if (prompt) {
     // x_n into the attention output's buffer, free until the attention runs
     hipLaunchKernelGGL(k_rmsnorm, dim3(rows), dim3(kThreads), 0, st, x, w->norm_w, eps, attn);
     OI2_CHECK_LAUNCH();
     ProjArgs p{};
-    p.x = attn;
-    p.rows = rows;
     p.w0 = w->wq;
     p.w1 = w->wk;
     p.w2 = w->wv;
@@ -940,15 +923,32 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
     p.sin = sin;
     p.counters = counters;
     p.n_counters = past + seq > kOneWgMax && !flash ? rows * n_kv : 0;
-    launch_proj(p, n_q + 2 * n_kv, st);
+    project(p, attn, rows, n_q + 2 * n_kv, st);
     OI2_CHECK_LAUNCH();
-  }
-  for (int r0 = 0; !prompt && r0 < rows; r0 += kMaxRows) {
-    const int rc = rows - r0 < kMaxRows ? rows - r0 : kMaxRows;
-    g.x = x + (size_t)r0 * kH;
-    g.row0 = r0;
-    g.counters = r0 == 0 ? counters : nullptr;
-    launch_gemv(g, rc, n_q + 2 * n_kv, st);
+  } else {
+    GemvArgs g{};
+    g.x = x;
+    g.norm_w = w->norm_w;
+    g.eps = eps;
+    g.w0 = w->wq;
+    g.w1 = w->wk;
+    g.w2 = w->wv;
+    g.blocks0 = n_q;
+    g.blocks1 = n_kv;
+    g.mode = 0;
+    g.q = qb;
+    g.q_width = n_q * kHd;
+    g.k_cache = k_cache;
+    g.v_cache = v_cache;
+    g.n_kv = n_kv;
+    g.cap = cache_cap;
+    g.past = past;
+    g.seq = seq;
+    g.cos = cos;
+    g.sin = sin;
+    g.counters = counters;
+    g.n_counters = rows * n_kv;
+    launch_gemv(g, rows, n_q + 2 * n_kv, st);
     OI2_CHECK_LAUNCH();
   }
 
@@ -1000,8 +1000,6 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
 
   if (prompt) {
     ProjArgs p{};
-    p.x = attn;
-    p.rows = rows;
     p.w0 = w->wo;
     p.blocks0 = kH / kHd;
     p.mode = 1;
@@ -1009,26 +1007,19 @@ int oi2_attn_forward(const uint16_t* x, int32_t batch, int32_t seq, const oi2_at
     p.out = out;
     p.residual = x_out ? x : nullptr;
     p.x_out = x_out;
-    launch_proj(p, kH / kHd, st);
-    OI2_CHECK_LAUNCH();
-    return OI2_OK;
+    project(p, attn, rows, kH / kHd, st);
+  } else {
+    GemvArgs o{};
+    o.x = attn;
+    o.w0 = w->wo;
+    o.blocks0 = kH / kHd;
+    o.mode = 1;
+    o.out = out;
+    o.residual = x_out ? x : nullptr;
+    o.x_out = x_out;
+    launch_gemv(o, rows, kH / kHd, st);
   }
-  GemvArgs o{};
-  o.norm_w = nullptr;
-  o.w0 = w->wo;
-  o.blocks0 = kH / kHd;
-  o.blocks1 = 0;
-  o.mode = 1;
-  o.out = out;
-  o.residual = x_out ? x : nullptr;
-  o.x_out = x_out;
-  for (int r0 = 0; r0 < rows; r0 += kMaxRows) {
-    const int rc = rows - r0 < kMaxRows ? rows - r0 : kMaxRows;
-    o.x = attn + (size_t)r0 * kH;
-    o.row0 = r0;
-    launch_gemv(o, rc, kH / kHd, st);
-    OI2_CHECK_LAUNCH();
-  }
+  OI2_CHECK_LAUNCH();
   return OI2_OK;
 }
 

@@ -24,14 +24,14 @@ __device__ __forceinline__ RopePair rope_f16(_Float16 x1, _Float16 x2, _Float16 
 // Rows of x times weight blocks of 128 rows (one head each): q / k / v with
 // RoPE, q to a buffer and k, v into the cache (mode 0), or o_proj (mode 1).
 struct ProjArgs {
-  const uint16_t* x;          // input rows (rows, H) fp16
-  int rows;
+  const uint16_t* x;          // this launch's input rows (rows, H) fp16
+  int rows, row0;             // their number, at most kProjMaxRows, and the first one's index in the call
   const uint8_t* w0;          // weight blocks of 128 rows (.., H), fp8 e4m3fn
   const uint8_t* w1;
   const uint8_t* w2;
   int blocks0, blocks1;       // 128-row blocks in w0 and w1; the rest are w2's
   int mode;
-  // mode 0
+  // mode 0: what follows is the whole call's
   uint16_t* q;                // (rows, n_q * 128)
   int q_width;                // n_q * 128
   uint16_t* k_cache;
@@ -47,6 +47,7 @@ struct ProjArgs {
   uint16_t* x_out;
 };
 
+constexpr int kProjMaxRows = 0x7FFFFFFF / (2 * 4096) / 128 * 128;   // 32-bit byte offsets into the rows, whole tiles
 void launch_proj(const ProjArgs& a, int n_heads, hipStream_t st);
 
 // Attention of (batch, seq) query rows over cache positions [0, past + seq).

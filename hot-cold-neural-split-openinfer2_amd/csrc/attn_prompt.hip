@@ -260,8 +260,8 @@ __global__ __launch_bounds__(256, KB == 64 ? 2 : 1) void k_proj(ProjArgs a, int 
   const bool rot = hb < a.blocks0 + a.blocks1;
 #pragma unroll
   for (int it = 0; it < kBM * 8 / 256; ++it) {
-    const int i = threadIdx.x + 256 * it, r = i >> 3, j = 8 * (i & 7), row = m0 + r;
-    if (row >= a.rows) break;
+    const int i = threadIdx.x + 256 * it, r = i >> 3, j = 8 * (i & 7), row = a.row0 + m0 + r;
+    if (m0 + r >= a.rows) break;
     u32x4 v0 = *reinterpret_cast<const u32x4*>(y0 + r * kHalfHead + j);
     u32x4 v1 = *reinterpret_cast<const u32x4*>(y1 + r * kHalfHead + j);
     if (a.mode == 1) {
@@ -382,8 +382,8 @@ __global__ __launch_bounds__(kFewThreads, 4) void k_proj_few(ProjArgs a) {
     s_r[w][l] = acc[nt];
     __syncthreads();
     // thread i < 128: row i / 8, pair i % 8
-    const int r = threadIdx.x >> 3, p = threadIdx.x & 7, row = 16 * nt + r, j = j0 + p;
-    if (r >= 16 || row >= a.rows) continue;
+    const int r = threadIdx.x >> 3, p = threadIdx.x & 7, row = a.row0 + 16 * nt + r, j = j0 + p;
+    if (r >= 16 || 16 * nt + r >= a.rows) continue;
     float y0 = 0.0f, y1 = 0.0f;
 #pragma unroll
     for (int k = 0; k < kFewWaves; ++k) {
@@ -753,6 +753,7 @@ __global__ __launch_bounds__(128 * NK, 4 / NK) void k_flash(FlashArgs a, int n_q
 //   512    37.4  20.4    31.3  26.8    32.8  28.1
 //   768    55.5  37.4    58.7  31.5    49.6  31.8
 //   1000   66.7  43.1    64.0  34.6    57.7  37.2
+static_assert(kH == 4096, "kProjMaxRows");
 void launch_proj(const ProjArgs& a, int n_heads, hipStream_t st) {
   if (a.rows <= 16 || (a.rows <= 32 && n_heads <= 64)) {
     if (a.rows <= 16) hipLaunchKernelGGL(k_proj_few<1>, dim3(8 * n_heads), dim3(kFewThreads), 0, st, a);

@@ -7,11 +7,14 @@ rel err 1e-2 and cosine >= 0.9999 of the float64 oracle over the same fp8
 weights and the same cache contents; cache positions below ``past`` are left
 bit for bit; the fused residual is exactly fp16(x + out).
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import oi2
+from oi2 import _lib
 from oracle import oracle as O
 from tests.gpu_helpers import EPS, assert_ffn_close
 
@@ -370,3 +373,34 @@ def test_a_token_gets_the_same_k_and_v_whichever_projection_runs(dev, rows):
         share = float((a != b[:, :, :n]).float().mean())
         print(f"[attn] {rows} rows: {share:.2%} of {name} differ from the call of {n}", flush=True)
         assert share <= 0.02, name
+
+
+def _forward(w, n_kv, x, cos, sin, k, v, past, causal, batch):
+    """oi2_attn_forward over caches of k's own capacity, through the C ABI."""
+    L, p = oi2.load_library(), "layer_000."
+    T, dev = x.shape[0] // batch, x.device
+    s = _lib.Attn(H // D, n_kv, *(w[p + n].data_ptr() for n in ("q_proj", "k_proj", "v_proj", "o_proj", "input_layernorm")))
+    nb = L.oi2_attn_workspace_bytes(batch, T, H // D, n_kv, past)
+    ws, out = torch.empty(nb, dtype=torch.uint8, device=dev), torch.empty_like(x)
+    _lib.check(L.oi2_attn_forward(x.data_ptr(), batch, T, ctypes.byref(s), EPS, cos.data_ptr(), sin.data_ptr(), k.data_ptr(),
+                                  v.data_ptr(), k.shape[2], past, int(causal), out.data_ptr(), None, ws.data_ptr(), nb,
+                                  _lib.stream_handle(dev)))
+    torch.cuda.synchronize()
+    return out
+
+
+def test_more_rows_than_one_projection_launch_addresses(dev):
+    """262146 sequences of one token, past the rows that one launch's 32-bit
+    offsets reach (a multiple of 128 below 2^31 / 8192): the last 130 rows equal
+    those of a call of their own, but for the order of the fp32 sums."""
+    n_kv, B, n = 4, 262016 + 130, 130
+    w = _weights(dev, n_kv, seed=101)
+    cos, sin = (t[7:].contiguous() for t in oi2.rope_tables(8, D, 1e6, device=dev))
+    x = torch.randn((B, H), generator=torch.Generator(device=dev).manual_seed(102), device=dev, dtype=torch.float16)
+    res = []
+    for rows in (x, x[-n:].contiguous(), x[:n].contiguous()):
+        k, v = (torch.full((rows.shape[0], n_kv, 1, D), 9.0, device=dev, dtype=torch.float16) for _ in range(2))
+        res.append((_forward(w, n_kv, rows, cos, sin, k, v, 0, True, rows.shape[0]), k, v))
+    for what, part, alone in (("last", slice(-n, None), res[1]), ("first", slice(0, n), res[2])):
+        for a, b in zip(res[0], alone):
+            assert_ffn_close(a[part].float().cpu().numpy(), b.float().cpu().numpy(), tol=2e-3, what=f"{what} rows")
