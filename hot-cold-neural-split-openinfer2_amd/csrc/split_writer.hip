@@ -139,7 +139,8 @@ __device__ __forceinline__ void section_frame(uint8_t* section, int layer, int e
   for (size_t i = body + t; i < total; i += kThreads) section[i] = 0;
 }
 
-// One launch: workgroup 0 frames the section, the next take the strided
+// One launch (per kMaxRecords records): workgroup 0 frames the section, the next
+// take the strided
 // vectors (8 per tiles x kGroups / kColGroups each; the longest ones first),
 // the rest one consecutive vector each.  Bound by memory: a 10752-record
 // section reads 528 MB and writes 69 MB in 139 us, 4.3 TB/s (a large copy
@@ -149,15 +150,15 @@ struct SectionArgs {
   QuantArgs q;
   int rows_v[3], cols_v[3], n_rows, n_cols;   // vectors by kind
   int tiles, per;                             // 64-record tiles, and per XCD
-  uint8_t* section;
-  int layer, expert;
+  uint8_t* section;                           // null: framed by another launch
+  int layer, expert, n;                       // n: the section's records (q.n the launch's)
   size_t body, total;
 };
 __global__ __launch_bounds__(kThreads) void k_quantize_section(SectionArgs a) {
   __shared__ float s_max[2][4][kWave];
   int b = blockIdx.x;
   if (b == 0) {
-    section_frame(a.section, a.layer, a.expert, a.q.n, a.body, a.total);
+    if (a.section) section_frame(a.section, a.layer, a.expert, a.n, a.body, a.total);
     return;
   }
   b -= 1;
@@ -173,6 +174,10 @@ __global__ __launch_bounds__(kThreads) void k_quantize_section(SectionArgs a) {
   b -= cols;
   quantize_row(a.q, b % a.q.n, a.rows_v[b / a.q.n]);
 }
+
+// A launch has at most 2^32 threads, which three workgroups a record would pass
+// at 5.6 million records.
+constexpr int kMaxRecords = 1 << 20;
 
 size_t section_bytes(int64_t n) {
   const size_t body = kHeader + (size_t)n * kRecBytes;
@@ -204,6 +209,7 @@ extern "C" int oi2_quantize_section(int32_t layer, int32_t expert, int32_t n, co
   sa.section = section;
   sa.layer = layer;
   sa.expert = expert;
+  sa.n = n;
   sa.body = (size_t)kHeader + (size_t)n * kRecBytes;
   sa.total = need;
   if (n > 0) {
@@ -218,20 +224,26 @@ extern "C" int oi2_quantize_section(int32_t layer, int32_t expert, int32_t n, co
       a.row_stride[m] = row_stride[m];
       a.elem_stride[m] = elem_stride[m];
     }
-    a.nids = nids;
-    a.rows = rows;
-    a.n = n;
-    a.records = section + kHeader;
     for (int m = 0; m < 3; ++m) {
       if (elem_stride[m] == 1) sa.rows_v[sa.n_rows++] = m;
       else sa.cols_v[sa.n_cols++] = m;
     }
     sa.q = a;
   }
-  sa.tiles = (n + kWave - 1) / kWave;
-  sa.per = (sa.tiles + 7) / 8;
-  const int64_t grid = 1 + (int64_t)sa.n_cols * (kGroups / kColGroups) * 8 * sa.per + (int64_t)sa.n_rows * n;
-  hipLaunchKernelGGL(k_quantize_section, dim3((unsigned)grid), dim3(kThreads), 0, st, sa);
-  OI2_CHECK_LAUNCH();
+  int r0 = 0;
+  do {                                         // once for an empty section, to frame it
+    const int nr = n - r0 < kMaxRecords ? n - r0 : kMaxRecords;
+    sa.q.n = nr;
+    sa.q.nids = nids + r0;
+    sa.q.rows = rows + r0;
+    sa.q.records = section + kHeader + (size_t)r0 * kRecBytes;
+    sa.tiles = (nr + kWave - 1) / kWave;
+    sa.per = (sa.tiles + 7) / 8;
+    const int grid = 1 + sa.n_cols * (kGroups / kColGroups) * 8 * sa.per + sa.n_rows * nr;
+    hipLaunchKernelGGL(k_quantize_section, dim3(grid), dim3(kThreads), 0, st, sa);
+    OI2_CHECK_LAUNCH();
+    sa.section = nullptr;
+    r0 += nr;
+  } while (r0 < n);
   return OI2_OK;
 }

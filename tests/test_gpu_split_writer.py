@@ -4,6 +4,7 @@ bytes are identical to the reference writer's -- the golden SHA-256 of the
 reference fixture file (tests/common.py:31-104, seed 0), the host writer
 over the same inputs at real geometry, and the oracle quantiser on crafted
 ties, zero groups, clamp-bound, fp16-subnormal and fp16-overflowing scales."""
+import ctypes
 import hashlib
 import json
 import os
@@ -13,6 +14,8 @@ import numpy as np
 import pytest
 import torch
 
+import oi2
+from oi2 import _lib
 from oi2 import format as fmt
 from oi2.split import ColdSectionWriter, quantize_section, quantize_section_rows, section_nbytes
 from oracle import oracle as O
@@ -128,3 +131,30 @@ def test_strided_vectors_match_the_host_writer(dev, n):
     sec = _run(3, 0, *t, rows.astype(np.int64), nids, (1, 1, 1), (width, width, width)).cpu().numpy()
     ref = fmt.section_bytes(3, fmt.build_records(nids, *[m.T[rows] for m in mats]))
     assert sec.tobytes() == ref
+
+
+@pytest.mark.parametrize("n,strided", [(64 * 16385, True), (64 * 87500, False)])
+def test_sections_past_one_launch(dev, n, strided):
+    """More records than one launch takes (2^20, and 5.6 million, whose
+    workgroups a single launch could not number): 64 neurons over and over, each
+    record as in a section of those 64."""
+    gen = torch.Generator(device=dev).manual_seed(5)
+    gate, up, down = (torch.randn((64, H), generator=gen, device=dev) * 0.02 for _ in range(3))
+    L = oi2.load_library()
+    if strided:
+        down = down.t().contiguous()
+    rs, es = (ctypes.c_int64 * 3)(H, H, 1 if strided else H), (ctypes.c_int64 * 3)(1, 1, 64 if strided else 1)
+
+    def section(count):
+        rows = torch.arange(count, device=dev, dtype=torch.int32) % 64
+        nids, out = rows.short(), torch.empty(int(L.oi2_section_bytes(count)), dtype=torch.uint8, device=dev)
+        _lib.check(L.oi2_quantize_section(3, 1, count, nids.data_ptr(), rows.data_ptr(), gate.data_ptr(), up.data_ptr(),
+                                          down.data_ptr(), ctypes.cast(rs, ctypes.c_void_p), ctypes.cast(es, ctypes.c_void_p),
+                                          out.data_ptr(), out.numel(), _lib.stream_handle(dev)))
+        torch.cuda.synchronize()
+        return out
+    want, got = section(64), section(n)
+    assert got[:16].cpu().numpy().tobytes() == np.array([3, 1], "<u2").tobytes() + np.array([n], "<u4").tobytes() + want[8:16].cpu().numpy().tobytes()
+    body = got[16:16 + n * 6400].view(n // 64, 64 * 6400)
+    same = all(bool((part == want[16:16 + 64 * 6400]).all()) for part in body.split(2000))
+    assert same and not got[16 + n * 6400:].any()
