@@ -92,6 +92,20 @@ def _rand_cache(dev, B, n_kv, past, seed):
     return k, v
 
 
+def _forward(w, n_kv, x, cos, sin, k, v, past, causal, batch):
+    """oi2_attn_forward over caches of k's own capacity, through the C ABI."""
+    L, p = oi2.load_library(), "layer_000."
+    T, dev = x.shape[0] // batch, x.device
+    s = _lib.Attn(H // D, n_kv, *(w[p + n].data_ptr() for n in ("q_proj", "k_proj", "v_proj", "o_proj", "input_layernorm")))
+    nb = L.oi2_attn_workspace_bytes(batch, T, H // D, n_kv, past)
+    ws, out = torch.empty(nb, dtype=torch.uint8, device=dev), torch.empty_like(x)
+    _lib.check(L.oi2_attn_forward(x.data_ptr(), batch, T, ctypes.byref(s), EPS, cos.data_ptr(), sin.data_ptr(), k.data_ptr(),
+                                  v.data_ptr(), k.shape[2], past, int(causal), out.data_ptr(), None, ws.data_ptr(), nb,
+                                  _lib.stream_handle(dev)))
+    torch.cuda.synchronize()
+    return out
+
+
 @pytest.mark.parametrize("B,past,n_kv", [(1, 5, 8), (1, 37, 8), (3, 300, 8), (1, 4095, 8), (3, 1000, 8), (2, 100, 32),
                                          (2, 129, 4), (1, 255, 16), (1, 1023, 8), (2, 1024, 8)])
 def test_decode_step_against_oracle(dev, B, past, n_kv):
@@ -114,8 +128,8 @@ def test_decode_step_against_oracle(dev, B, past, n_kv):
 def test_long_spans_in_looping_splits(dev, B, T, past, n_kv):
     """Spans whose 256-position splits number at least 208: the last split of
     one position, of all 256 and of most of them, one split fewer (one-shot
-    splits), query groups of 1, 2, 4 and 8; keys that grow along the span, so
-    every chunk raises the running max."""
+    splits), query groups of 1, 2, 4 and 8; keys that grow along the span.  A
+    position hardly weighs here: the test after this one gives each split's own."""
     w = _weights(dev, n_kv, seed=past + n_kv)
     attn = oi2.GroupedQueryAttention(0, w, _cfg(n_kv))
     cos, sin = oi2.rope_tables(past + T, D, 10000.0, device=dev)
@@ -124,6 +138,103 @@ def test_long_spans_in_looping_splits(dev, B, T, past, n_kv):
     k, v = _rand_cache(dev, B, n_kv, past, seed=past)
     k *= torch.linspace(0.1, 2.0, past, device=dev).half()[:, None]
     _check_step(attn, w, n_kv, x, cos[past:], sin[past:], (k, v), f"B={B} T={T} past={past} n_kv={n_kv}")
+
+
+def _row_err(y, ref):
+    """Largest error of each row (last axis) over the row's largest value."""
+    y, ref = np.asarray(y, np.float64), np.asarray(ref, np.float64)
+    return np.abs(y - ref).max(-1) / np.abs(ref).max(-1)
+
+
+@pytest.mark.parametrize("B,T,past,n_kv", [(8, 1, 1024, 8), (1, 1, 8192, 8), (1, 1, 6400, 8), (1, 1, 6399, 8), (4, 1, 1280, 16),
+                                           (2, 1, 1055, 32), (1, 5, 2040, 8), (7, 1, 1792, 4), (1, 1, 1500, 8), (1, 1, 900, 8)])
+def test_every_split_of_a_long_span_counts(dev, B, T, past, n_kv):
+    """Scores that rise by 4 along the span, so that every chunk of every split
+    raises the running max, and about one position in each 64 (every offset,
+    the ends of the span, the last split's first position) whose v makes up for
+    its probability: each adds 1/64 to the output, whose rows are compared one
+    by one.  Half the weight of one of them is past the bar, 3 times the fp16
+    rounding of the output (2^-11 of the largest value) and as much again for
+    the fp32 exponentials and sums; the oracle with the last position, or the
+    last split's first, left out shows that the bar sees one."""
+    G, n = 32 // n_kv, past + T
+    g = torch.Generator(device=dev).manual_seed(past + n_kv)
+    p = "layer_000."
+
+    def cols(rows, count, value=1.0):
+        w = torch.zeros((rows, H), device=dev)
+        w[:, :count] = value * 2.0 ** -9
+        return w.to(torch.float8_e4m3fn)
+    # x_n = 1: q = 1 and k = 0.36 in every dim, v = +-32; out is the attention itself
+    sign = torch.where(torch.rand((n_kv * D, 1), generator=g, device=dev) < 0.5, -1.0, 1.0)
+    w = {p + "q_proj": cols(H, 512), p + "k_proj": cols(n_kv * D, 184), p + "v_proj": cols(n_kv * D, 512, 32.0 * sign),
+         p + "o_proj": torch.eye(H, device=dev).to(torch.float8_e4m3fn), p + "input_layernorm": torch.ones(H, device=dev).half()}
+    cos, sin = torch.ones((T, D // 2), device=dev), torch.zeros((T, D // 2), device=dev)
+    x = torch.ones((B, T, H), device=dev).half()
+    t = torch.linspace(0.0, 0.35, past, device=dev).half()
+    k = t[:, None].expand(B, n_kv, past, D).contiguous()
+    prob = torch.softmax(torch.cat([t.double(), torch.full((T,), 184 / 512, device=dev).double()]) * D ** 0.5, 0)
+    at = (torch.arange(0, past, 64, device=dev) + 37 * torch.arange(0, (past + 63) // 64, device=dev) % 64).clamp(max=past - 1)
+    last = (n - 1) // 256 * 256
+    at = torch.cat([at, torch.tensor([0, past - 1, min(last, past - 1)], device=dev)]).unique()
+    v = torch.randn((B, n_kv, past, D), generator=g, device=dev)
+    v[:, :, at] = torch.where(torch.rand((B, n_kv, at.numel(), D), generator=g, device=dev) < 0.5, -1.0, 1.0) \
+        * (1 / 64 / prob[at]).float()[:, None]
+    out, (k, v) = oi2.GroupedQueryAttention(0, w, _cfg(n_kv))(x, cos, sin, (k, v.half()))
+    bar = 3 * 2.0 ** -10
+    kn, vn = k.double().cpu().numpy(), v.double().cpu().numpy()
+
+    def reference(keep):
+        q = np.ones((B, 32, T, D))
+        return O.attention_core(q, kn[:, :, keep], vn[:, :, keep], causal=False).transpose(0, 2, 1, 3)
+    every = np.arange(n)
+    ref = reference(every)
+    err = _row_err(out.float().cpu().numpy().reshape(B, T, 32, D), ref)
+    print(f"[attn] B={B} T={T} past={past} n_kv={n_kv}: row error {err.max():.1e}, bar {bar:.1e}", flush=True)
+    assert err.max() <= bar
+    for lost in {n - 1, min(last, past - 1)}:
+        assert _row_err(reference(every[every != lost]), ref).min() > 2 * bar
+
+
+def _weights_out_is_attention(dev, n_kv, seed):
+    w = _weights(dev, n_kv, seed)
+    w["layer_000.o_proj"] = torch.eye(H, device=dev).to(torch.float8_e4m3fn)
+    return w
+
+
+@pytest.mark.parametrize("T,past,n_kv", [(400, 0, 8), (700, 0, 16), (3, 100, 8), (3, 1100, 8), (9, 60, 8), (70, 100, 8), (130, 1100, 4),
+                                         (600, 33, 8)])
+def test_causal_rows_see_their_own_position_and_no_later_one(dev, T, past, n_kv):
+    """Causal rows at and beside the edges of tiles of rows and positions, each
+    against the oracle's attention over exactly the positions up to its own,
+    also behind a cache (which the C ABI allows and the engine does not ask
+    for); the oracle with one position fewer or more shows that the bar, 5e-3 of
+    the row's largest value, tells them apart."""
+    w = _weights_out_is_attention(dev, n_kv, seed=111)
+    n = past + T
+    cos, sin = (t[past:].contiguous() for t in oi2.rope_tables(n, D, 1e6, device=dev))
+    x = torch.randn((T, H), generator=torch.Generator(device=dev).manual_seed(112), device=dev).half()
+    k, v = (torch.zeros((1, n_kv, n, D), device=dev).half() for _ in range(2))
+    if past:
+        for t, r in zip((k, v), _rand_cache(dev, 1, n_kv, past, seed=113)):
+            t[:, :, :past] = r
+    out = _forward(w, n_kv, x, cos, sin, k, v, past, True, 1).float().cpu().numpy().reshape(T, 32, D)
+    kn, vn = k.double().cpu().numpy(), v.double().cpu().numpy()
+    xn = O.rmsnorm(x.double().cpu().numpy(), w["layer_000.input_layernorm"].double().cpu().numpy(), EPS).astype(np.float16)
+    q = (xn.astype(np.float64) @ w["layer_000.q_proj"].double().cpu().numpy().T).astype(np.float16).astype(np.float64)
+    q = O.apply_rope(q.reshape(1, T, 32, D).transpose(0, 2, 1, 3), *(t.half().double().cpu().numpy() for t in (cos, sin)))
+    q = q.astype(np.float16).astype(np.float64)
+    rows = sorted({r for e in (0, 32, 63, 64, 127, 128, 255, 256, 383, 512, T - 1) for r in (e - 1, e, e + 1) if 0 <= r < T})
+    for r in rows:
+        see = past + r + 1
+        one = lambda m: O.attention_core(q[:, :, r:r + 1], kn[:, :, :m], vn[:, :, :m], causal=False)[0, :, 0]
+        ref = one(see)
+        err = _row_err(out[r], ref).max()
+        assert err <= 5e-3, (r, err)
+        for m in (see - 1, see + 1):
+            if 0 < m <= n:
+                assert _row_err(one(m), ref).max() > 1e-2
+    print(f"[attn] T={T} past={past} n_kv={n_kv}: {len(rows)} rows", flush=True)
 
 
 def test_prefill_then_decode_like_the_engine(dev):
@@ -373,20 +484,6 @@ def test_a_token_gets_the_same_k_and_v_whichever_projection_runs(dev, rows):
         share = float((a != b[:, :, :n]).float().mean())
         print(f"[attn] {rows} rows: {share:.2%} of {name} differ from the call of {n}", flush=True)
         assert share <= 0.02, name
-
-
-def _forward(w, n_kv, x, cos, sin, k, v, past, causal, batch):
-    """oi2_attn_forward over caches of k's own capacity, through the C ABI."""
-    L, p = oi2.load_library(), "layer_000."
-    T, dev = x.shape[0] // batch, x.device
-    s = _lib.Attn(H // D, n_kv, *(w[p + n].data_ptr() for n in ("q_proj", "k_proj", "v_proj", "o_proj", "input_layernorm")))
-    nb = L.oi2_attn_workspace_bytes(batch, T, H // D, n_kv, past)
-    ws, out = torch.empty(nb, dtype=torch.uint8, device=dev), torch.empty_like(x)
-    _lib.check(L.oi2_attn_forward(x.data_ptr(), batch, T, ctypes.byref(s), EPS, cos.data_ptr(), sin.data_ptr(), k.data_ptr(),
-                                  v.data_ptr(), k.shape[2], past, int(causal), out.data_ptr(), None, ws.data_ptr(), nb,
-                                  _lib.stream_handle(dev)))
-    torch.cuda.synchronize()
-    return out
 
 
 def test_more_rows_than_one_projection_launch_addresses(dev):
