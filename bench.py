@@ -820,7 +820,7 @@ def measure_decode_step(ffn_layers_syn, thr, dev, ctx=512, reps=20, seed=7):
         out[name] = {"us_per_token": us, "us_per_layer": us / N_LAYERS, "tok_s": 1e6 / us}
     stack.close()
     out["path"] = ("DecoderStep: GroupedQueryAttention (3 kernels per layer) + FFN per layer as the "
-                   "drop-in SparseFFNLayer (predictor 3 kernels, FFN 3) or DecodeStack.layer "
+                   "drop-in SparseFFNLayer (predictor 3 kernels, FFN 2) or DecodeStack.layer "
                    "(3 kernels with the next layer's prediction fused); one graph per token")
     return out
 

@@ -308,15 +308,20 @@ __global__ __launch_bounds__(kThreads) void k_attn_gemv(GemvArgs a) {
 // its reductions over lanes, waves and splits follow every 128 positions; once
 // workgroups of 256 positions nearly fill the chip, half as many of them hide
 // more (whole layer, one-shot and LOOP, us: n_kv 8, 8 sequences at 2000
-// positions 42.5 and 39.8, 2 at 4000 30.8 and 28.7, 1 at 8000 32.0 and 28.2;
-// n_kv 16, 4 at 2000 37.0 and 34.8; n_kv 32, 1 at 4000 35.7 and 31.4).  512
-// positions per workgroup: 43.2, 32.4, 31.0, 35.3, 30.8.  8 query heads per
-// kv head take chunks of half the length (n_kv 4: 16 sequences at 2000 59.5
-// and 51.8, 8 at 3000 51.3 and 48.7; with the others' chunks, 55.4).
+// positions 41.6 and 37.9, 2 at 4000 28.8 and 26.2, 1 at 8000 29.9 and 25.4;
+// n_kv 16, 4 at 2000 35.0 and 33.6; n_kv 32, 1 at 4000 34.8 and 30.3).  With
+// 512 positions per workgroup 37.6, 33.1 and 28.6 where that leaves 208 of them
+// (the first and the last two).  8 query heads per kv head take chunks of half
+// the length (n_kv 4: 16 sequences at 2000 54.0 one-shot, 49.8; 8 at 3000 44.0,
+// 47.6): a choice made, like kLoopMinWgs, with loads that clamped the positions
+// past the span to the last one, an address computation each; with the others'
+// chunks those two now take 48.2 and 45.3.
 constexpr int kLoopSpan = 256;           // positions per workgroup
-// 216 workgroups (n_kv 8, one sequence at 6900 positions) 30.5 one-shot, 27.6;
-// 224 (n_kv 16, 2 at 1700) 26.7, 25.6; 192 (n_kv 8, 3 at 2000) 27.9, 28.2; 168
-// (3 at 1700) 27.7, 28.3.
+// With the clamped loads 216 workgroups (n_kv 8, one sequence at 6900 positions)
+// took 30.5 one-shot, 27.6 LOOP; 224 (n_kv 16, 2 at 1700) 26.7, 25.6; 192 (n_kv
+// 8, 3 at 2000) 27.9, 28.2; 168 (3 at 1700) 27.7, 28.3.  With the present ones
+// LOOP is the faster below the line too, which has stayed: 192 27.7, 25.1; 168
+// 26.9, 25.2; 128 (1 at 4000) 22.4, 21.6; n_kv 4, 1 at 4000 (64) 40.6, 25.2.
 constexpr int kLoopMinWgs = 208;
 constexpr int loop_steps(int G) { return G == 8 ? 2 : 4; }
 template <int G, int STEPS, bool LOOP>

@@ -439,11 +439,14 @@ __global__ __launch_bounds__(kFewThreads, 4) void k_proj_few(ProjArgs a) {
 // Probabilities stay 32-bit: p 2^10 = hi + lo in two fp16 parts (hi truncated,
 // lo the rest, at least 21 bits; the 2^10 keeps lo of small p out of the
 // subnormals and cancels in the division by the sum), two MFMAs per fragment.
+// What both truncate is below 2^-21 p or 2^-34 (the sum keeps it): at most
+// n 2^-34 of the output over n positions, and the layer's error against float64
+// is the fp32 kernels' (512 rows 7.8e-4 with either).
 //
 // What bounds it: the chain of one tile (scores, max, probabilities, output:
 // 24 MFMAs and ~200 vector instructions a wave) and, causal, the longest row
-// tile's chain of tiles.  512 rows 17 us (one workgroup per query row and
-// head, the single-token kernel: 134), 1300 rows 38 us (split kernel: 1078).
+// tile's chain of tiles.  512 rows 16 us (one workgroup per query row and
+// head, the single-token kernel: 134), 1300 rows 39 us (split kernel: 1078).
 // Reading a tile's eight K fragments ahead of its MFMAs changed nothing.
 //
 // K goes to LDS by DMA; V through registers, 4 positions x 8 dims a thread,
@@ -772,7 +775,7 @@ void launch_proj(const ProjArgs& a, int n_heads, hipStream_t st) {
 
 // Four position parts (eight waves, 128 positions a tile) while every
 // workgroup has a CU to itself, else two (two workgroups a CU): 1300 rows, 672
-// workgroups, 38.5 against 54.3 us; 9 rows over 4000 positions, 32 workgroups,
+// workgroups, 38.6 against 49.1 us; 9 rows over 4000 positions, 32 workgroups,
 // the layer 90 against 110 us.
 void launch_flash(const FlashArgs& a, hipStream_t st) {
   const int n_qt = (a.seq + kFQ - 1) / kFQ, wgs = kH / kHeadDim * n_qt * a.batch;

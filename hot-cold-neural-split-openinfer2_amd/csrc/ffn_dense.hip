@@ -19,8 +19,10 @@
 // them.  Products on the matrix cores: fp16 weights with the fp16 x as they
 // are (16x16x32 f16, exact products), everything else in fp32 (16x16x4 f32):
 // bf16 and fp32 weights, and the whole down product, whose h stays fp32.
-// 13 tokens, 3584 fp16 hot and 538 fp32 cold neurons (115 MB of weights): one
-// GEMV pass per four tokens, four launches each, took 184 us, these two 43.
+// 13 tokens, 3584 fp16 hot and 538 fp32 cold neurons (115 MB of weights), the
+// whole Python call with its cast of the fp32 y to x's type (a third launch):
+// with one GEMV pass per four tokens, four launches each, 184 us, with these two
+// (24 + 18) 43.
 #include "capi_util.h"
 #include "ffn_kernels.h"
 

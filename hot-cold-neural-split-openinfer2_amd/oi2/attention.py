@@ -51,7 +51,9 @@ def _fp8_bytes(w: torch.Tensor, shape, what: str, device) -> torch.Tensor:
 
 class GroupedQueryAttention(torch.nn.Module):
     """engine.py:63-125 on the GPU: RMSNorm, q/k/v projections, RoPE, KV
-    append, grouped attention and o_proj as three HIP kernels."""
+    append, grouped attention and o_proj as three HIP kernels, four from 6
+    token rows on.  RoPE rounds alike in all of them; the order of the fp32
+    sums, and with it a rare last bit, depends on the rows that share a call."""
 
     def __init__(self, layer_idx: int, weights: dict, cfg: dict, device=None):
         super().__init__()

@@ -259,7 +259,7 @@ def test_prefill_then_decode_like_the_engine(dev):
 
 
 def test_rows_beyond_one_launch_and_noncausal_chunk(dev):
-    """12 query rows (two projection launches of up to 8 rows), causal
+    """12 query rows (past the five that one GEMV launch takes), causal
     prefill; then a 3-token chunk over a cache, which the reference runs
     non-causally (is_causal is False whenever a cache is given,
     engine.py:121)."""
